@@ -487,7 +487,8 @@ def main():
     ap.add_argument("--geometry-config", default=None,
                     help="BVH width, traversal stack, waves per SIMD of the mesh frames (skips their tuner), e.g. 2,0,8")
     ap.add_argument("--geometry-stack", type=int, default=None,
-                    help="BVH traversal stack of the mesh frames: 0 private, 16/24/32 LDS (no tuning)")
+                    help="BVH traversal stack of the mesh frames: 0 the 4-wide walk, 16/24/32 the binary walk with that "
+                         "many entries in LDS (no tuning)")
     ap.add_argument("--batch-config", default=None,
                     help="chunk,stack,wpe,blocks_per_cu,layout of the batched and served forms (no tuning)")
     ap.add_argument("--serve-config", default=None,
@@ -572,7 +573,7 @@ def main():
         w = 6                               # 17 / 18 act as 16 beyond one bricked volume and isovalue
     bs = kcfg[1].value if (one and w == 6 and kcfg[1].value in (64, 128)) else 256
     roof["kernel"] = ("k_trace_pl<1>" if k == 1 else
-                      "k_trace<1,false,%d,%d,0,0,%d,%d>" % (w, sm, 1 if one else 8, bs))
+                      "k_trace<1,false,%d,%d,%d,%d>" % (w, sm, 1 if one else 8, bs))
     roof["volume_layout"] = lay
     roof["kernel_ms_per_launch"] = round(tr_ms / max(1, tr_n), 4)
     roof["alg_bytes_per_launch"] = int(alg_bytes / max(1, tr_n))

@@ -23,9 +23,8 @@ import ctypes as C
 
 DEFAULT_CANDIDATES = ([(0, 256, 32), (15, 256, 32), (16, 256, 32)] +
                       [(1, chunk, refill) for chunk in (128, 256) for refill in (16, 32)])
-# BVH traversal stacks of geometry-only traces: private memory (64 entries) or
-# 16 / 24 / 32 entries in LDS (a model deeper than the stack keeps the private one)
-GEOMETRY_STACKS = [0, 16, 24, 32]
+# traversal stack entries in LDS of the binary BVH walk (deeper ones in private memory)
+GEOMETRY_STACKS = [16, 24, 32]
 
 
 def _trace_ms(L):
@@ -60,9 +59,9 @@ def tune_trace(L, render_once, candidates=None, reps=2):
 
 def geometry_candidates(stacks=None):
     """(BVH width, traversal stack entries, waves per SIMD) of the geometry
-    tuner: both widths over the stacks at the compiler's occupancy, plus the
-    binary private-stack walk at 8 waves per SIMD."""
-    return [(w, s, 0) for w in (4, 2) for s in (stacks or GEOMETRY_STACKS)] + [(2, 0, 8)]
+    tuner: the 4-wide walk, the binary one over the stacks, and the binary one
+    at 8 waves per SIMD."""
+    return [(4, 0, 0)] + [(2, s, 0) for s in (stacks or GEOMETRY_STACKS)] + [(2, 0, 8)]
 
 
 def tune_geometry_stack(L, render_once, stacks=None, reps=2):

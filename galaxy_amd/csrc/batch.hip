@@ -102,11 +102,11 @@ __device__ __forceinline__ int chunk_layout(const TraceParams &P) { return sm_of
 template <int SM, int MI>
 __device__ __forceinline__ unsigned long long render_chunk(const TraceParams &P, const RayList_ispc &R,
                                                            const BatchChunk &ch, const float (*col)[3 * GXY_TF_MAX],
-                                                           const float (*op)[GXY_TF_MAX],
-                                                           PrivStack<GXY_BVH_STACK> &pstack) {
+                                                           const float (*op)[GXY_TF_MAX]) {
   unsigned long long n = 0;
+  NoStack stack;
   for (int k = threadIdx.x & 63; k < ch.count; k += 64)
-    n += trace_one<1, false, PrivStack<GXY_BVH_STACK>, SM, 0, MI>(P, R, ch.start + k, col, op, pstack);
+    n += trace_one<1, false, SM, MI>(P, R, ch.start + k, col, op, stack);
   return n;
 }
 // (bricked volumes with more than one isovalue take the 64-bit variants,
@@ -114,17 +114,16 @@ __device__ __forceinline__ unsigned long long render_chunk(const TraceParams &P,
 __device__ __forceinline__ unsigned long long render_chunk_any(const TraceParams &P, const RayList_ispc &R,
                                                                const BatchChunk &ch, int lay,
                                                                const float (*col)[3 * GXY_TF_MAX],
-                                                               const float (*op)[GXY_TF_MAX],
-                                                               PrivStack<GXY_BVH_STACK> &pstack) {
+                                                               const float (*op)[GXY_TF_MAX]) {
   const bool one = P.vv[0].nIso <= 1;
-  if (one && lay == 4) return render_chunk<4, 1>(P, R, ch, col, op, pstack);
-  if (one && lay == 12) return render_chunk<12, 1>(P, R, ch, col, op, pstack);
-  if (one && lay == 8) return render_chunk<8, 1>(P, R, ch, col, op, pstack);
-  if (one && lay == 16) return render_chunk<16, 1>(P, R, ch, col, op, pstack);
-  if (lay == 8 || lay == 16) return render_chunk<16, GXY_MAX_ISO>(P, R, ch, col, op, pstack);
-  if (lay == 4 || lay == 12) return render_chunk<12, GXY_MAX_ISO>(P, R, ch, col, op, pstack);
-  if (lay == 1) return render_chunk<1, GXY_MAX_ISO>(P, R, ch, col, op, pstack);
-  return render_chunk<0, GXY_MAX_ISO>(P, R, ch, col, op, pstack);
+  if (one && lay == 4) return render_chunk<4, 1>(P, R, ch, col, op);
+  if (one && lay == 12) return render_chunk<12, 1>(P, R, ch, col, op);
+  if (one && lay == 8) return render_chunk<8, 1>(P, R, ch, col, op);
+  if (one && lay == 16) return render_chunk<16, 1>(P, R, ch, col, op);
+  if (lay == 8 || lay == 16) return render_chunk<16, GXY_MAX_ISO>(P, R, ch, col, op);
+  if (lay == 4 || lay == 12) return render_chunk<12, GXY_MAX_ISO>(P, R, ch, col, op);
+  if (lay == 1) return render_chunk<1, GXY_MAX_ISO>(P, R, ch, col, op);
+  return render_chunk<0, GXY_MAX_ISO>(P, R, ch, col, op);
 }
 
 // The sampler rays of one chunk (samples and ray passes into acc).
@@ -218,17 +217,16 @@ __global__ __launch_bounds__(GXY_BLOCK) __attribute__((amdgpu_waves_per_eu(WPE >
 void k_btrace(BatchArgs A) {
   __shared__ float s_col[BWAVES][1][3 * GXY_TF_MAX];
   __shared__ float s_op[BWAVES][1][GXY_TF_MAX];
-  __shared__ int s_stack[STK > 0 ? STK : 1][GXY_BLOCK];
+  constexpr int NL = STK > 0 ? STK : GXY_LDS_STACK;
+  __shared__ int s_stack[NL][GXY_BLOCK];
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int nc = *A.nin;
   unsigned long long acc[BS_COUNT];
 #pragma unroll
   for (int k = 0; k < BS_COUNT; k++) acc[k] = 0;
   int cur_tf = -1;
-  PrivStack<GXY_BVH_STACK> pstack;
-  LdsStack<(STK > 0 ? STK : 1)> lstack;
-  lstack.base = &s_stack[0][threadIdx.x];
-  lstack.stride = GXY_BLOCK;
+  HybStack<NL, GXY_BLOCK> stack;
+  stack.base = &s_stack[0][threadIdx.x];
   for (;;) {
     int c = 0;
     if (lane == 0) c = atomicAdd(A.head, 1);
@@ -248,15 +246,10 @@ void k_btrace(BatchArgs A) {
       sample_chunk_any(A, P, R, ch, lay, xyz, pc, cap, acc);
     } else if (P.has_model) {
       acc[BS_RAYS] += lane < ch.count ? (ch.count - 1 - lane) / 64 + 1 : 0;
-      const bool wide = P.model.wide != 0;
+      const bool wide = P.model.wide == 1 || (P.model.wide == 2 && STK == 0);
       for (int k = lane; k < ch.count; k += 64) {
-        if (STK > 0) {
-          if (wide) acc[BS_SAMPLES] += trace_one<0, true, decltype(lstack), -1, 4>(P, R, ch.start + k, s_col[w], s_op[w], lstack);
-          else acc[BS_SAMPLES] += trace_one<0, true, decltype(lstack), -1, 2>(P, R, ch.start + k, s_col[w], s_op[w], lstack);
-        } else {
-          if (wide) acc[BS_SAMPLES] += trace_one<0, true, decltype(pstack), -1, 4>(P, R, ch.start + k, s_col[w], s_op[w], pstack);
-          else acc[BS_SAMPLES] += trace_one<0, true, decltype(pstack), -1, 2>(P, R, ch.start + k, s_col[w], s_op[w], pstack);
-        }
+        if (wide) trace_geom_one<decltype(stack), 4>(P, R, ch.start, k, stack);
+        else trace_geom_one<decltype(stack), 2>(P, R, ch.start, k, stack);
       }
     } else {
       acc[BS_RAYS] += lane < ch.count ? (ch.count - 1 - lane) / 64 + 1 : 0;
@@ -267,7 +260,7 @@ void k_btrace(BatchArgs A) {
         wave_lds_sync();
         cur_tf = ds;
       }
-      acc[BS_SAMPLES] += render_chunk_any(P, R, ch, lay, s_col[w], s_op[w], pstack);
+      acc[BS_SAMPLES] += render_chunk_any(P, R, ch, lay, s_col[w], s_op[w]);
     }
   }
   // lane sums of the sample and ray-pass counts
@@ -286,7 +279,8 @@ void k_btrace_kind(BatchArgs A) {
   constexpr int TFW = KIND == 0 ? BWAVES : 1;
   __shared__ float s_col[TFW][1][3 * GXY_TF_MAX];
   __shared__ float s_op[TFW][1][GXY_TF_MAX];
-  __shared__ int s_stack[(KIND == 1 && STK > 0) ? STK : 1][GXY_BLOCK];
+  constexpr int NL = KIND != 1 ? 1 : STK > 0 ? STK : GXY_LDS_STACK;
+  __shared__ int s_stack[NL][GXY_BLOCK];
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int nk = A.kcount[KIND];
   const int *idx = A.kidx + (size_t)KIND * A.kcap;
@@ -294,10 +288,8 @@ void k_btrace_kind(BatchArgs A) {
 #pragma unroll
   for (int k = 0; k < BS_COUNT; k++) acc[k] = 0;
   int cur_tf = -1;
-  PrivStack<GXY_BVH_STACK> pstack;
-  LdsStack<((KIND == 1 && STK > 0) ? STK : 1)> lstack;
-  lstack.base = &s_stack[0][threadIdx.x];
-  lstack.stride = GXY_BLOCK;
+  HybStack<NL, GXY_BLOCK> stack;
+  stack.base = &s_stack[0][threadIdx.x];
   for (;;) {
     int q = 0;
     if (lane == 0) q = atomicAdd(A.khead + KIND, 1);
@@ -317,15 +309,10 @@ void k_btrace_kind(BatchArgs A) {
       sample_chunk_any(A, P, R, ch, lay, xyz, pc, cap, acc);
     } else if (KIND == 1) {
       acc[BS_RAYS] += lane < ch.count ? (ch.count - 1 - lane) / 64 + 1 : 0;
-      const bool wide = P.model.wide != 0;
+      const bool wide = P.model.wide == 1 || (P.model.wide == 2 && STK == 0);
       for (int k = lane; k < ch.count; k += 64) {
-        if (STK > 0) {
-          if (wide) acc[BS_SAMPLES] += trace_one<0, true, decltype(lstack), -1, 4>(P, R, ch.start + k, s_col[0], s_op[0], lstack);
-          else acc[BS_SAMPLES] += trace_one<0, true, decltype(lstack), -1, 2>(P, R, ch.start + k, s_col[0], s_op[0], lstack);
-        } else {
-          if (wide) acc[BS_SAMPLES] += trace_one<0, true, decltype(pstack), -1, 4>(P, R, ch.start + k, s_col[0], s_op[0], pstack);
-          else acc[BS_SAMPLES] += trace_one<0, true, decltype(pstack), -1, 2>(P, R, ch.start + k, s_col[0], s_op[0], pstack);
-        }
+        if (wide) trace_geom_one<decltype(stack), 4>(P, R, ch.start, k, stack);
+        else trace_geom_one<decltype(stack), 2>(P, R, ch.start, k, stack);
       }
     } else {
       acc[BS_RAYS] += lane < ch.count ? (ch.count - 1 - lane) / 64 + 1 : 0;
@@ -336,7 +323,7 @@ void k_btrace_kind(BatchArgs A) {
         wave_lds_sync();
         cur_tf = ds;
       }
-      acc[BS_SAMPLES] += render_chunk_any(P, R, ch, lay, s_col[w % TFW], s_op[w % TFW], pstack);
+      acc[BS_SAMPLES] += render_chunk_any(P, R, ch, lay, s_col[w % TFW], s_op[w % TFW]);
     }
   }
   acc[BS_SAMPLES] = wave_sum_u64(acc[BS_SAMPLES]);

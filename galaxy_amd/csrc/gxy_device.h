@@ -128,7 +128,8 @@ struct DModel {
   const BVH4Node *snodes4;
   const BVH4Node *cnodes4;
   int depth4;           // deepest leaf of either 4-wide tree
-  int wide;             // traverse the 4-wide trees
+  int wide;             // 4-wide trees: 0 not walked, 1 asked for (BVH width 4), 2 walked unless a
+                        // setting of the binary walk is given (BVH width 2)
 };
 
 // Per-geometry shading data (DataDrivenTriangleMesh_postIntersect,

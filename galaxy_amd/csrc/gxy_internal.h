@@ -43,16 +43,24 @@ struct CameraParams {
 };
 
 // wpe: occupancy variant of the volume-only kernel (0 none, 5 or 6 waves/SIMD);
-// stack: BVH traversal stack of geometry-only launches (0: 64 entries in
-// private memory; 16, 24, 32: entries in LDS, used when the tree fits)
-// gwaves: 8 asks for 8 waves per SIMD (64 VGPRs) in the binary private-stack geometry walks (with or without
-// path lines), 0 the compiler's choice
+// stack, gwaves: settings of the binary geometry walk (stack entries in LDS 16,
+// 24 or 32, waves per SIMD 8); 0 and 0: the walk launch_trace_geom chooses
 // bs: work-items per workgroup of the one-bricked-volume, one-isovalue march
 // at 6 waves per SIMD (64, 128 or 256; GXY_BLOCK elsewhere):
 // trace_block_size(P, wpe, bs) is the size a launch uses
 hipError_t launch_trace(const TraceParams &P, const RayList_ispc &R, int n, int wpe, int stack, hipStream_t s,
                         int gwaves = 0, int bs = GXY_BLOCK);
 int trace_block_size(const TraceParams &P, int wpe, int bs);
+// the same for geometry without volumes (launch_trace calls it)
+hipError_t launch_trace_geom(const TraceParams &P, const RayList_ispc &R, int n, int stack, int gwaves,
+                             hipStream_t s);
+// Whether the 4-wide walk can take trees of this many levels, inner nodes and
+// primitives: it keeps at most three stack entries per level and the sentinel
+// (its stack holds GXY_LDS_STACK + GXY_STACK_OVER = 80 entries, trace_dev.h) and
+// addresses nodes (128 B) and primitives (at most 36 B) with 32-bit offsets.
+inline bool wide_walk_fits(int depth4, int nodes4, int prims) {
+  return 3 * depth4 + 2 <= 80 && nodes4 < (1 << 25) && prims < (1 << 26);
+}
 hipError_t launch_sampler(const TraceParams &P, const RayList_ispc &R, int n, hipStream_t s);
 // Persistent-lane trace for volume-only visualizations (1..4 volumes): each
 // wave owns `chunk` consecutive rays; idle lanes are refilled when at least

@@ -101,10 +101,10 @@ struct Runtime {
   int trace_kind = 0, trace_chunk = 256, trace_refill = 32, trace_wpe = 0;
   int ao_pcg = 0;          // AO directions: 0 the UV table (reference), 1 PCG32 streams
   unsigned ao_seed = 0;
-  int geom_stack = 0;           // BVH traversal stack of geometry-only traces (0 private, or LDS entries)
+  int geom_stack = 0;           // 16 / 24 / 32: binary walks with that many stack entries in LDS
   int occlusion = 1;            // rank loops: shadow/AO rays of volume-free scenes stop at their first hit
-  int bvh_width = 2;            // traverse the binary trees (2) or the 4-wide ones (4)
-  int geom_waves = 0;           // binary private-stack walks: 0 the compiler's occupancy, 8 waves per SIMD
+  int bvh_width = 2;            // 4: the 4-wide walk; 2: the same, or the binary one with geom_stack / geom_waves
+  int geom_waves = 0;           // 8: binary walks at 8 waves per SIMD
   float *uv = nullptr;          // AO direction tables U[256], V[256] (device)
   // device address of the static scratch array of the allocation-free spawn
   // offsets, per device (taken once, with that device current, at set-up)
@@ -441,6 +441,7 @@ struct ModelObj {
   int *hit_geom = nullptr, *hit_prim = nullptr;
   int tnodes = 0, snodes = 0, tdepth = 0, sdepth = 0, tdepth4 = 0, sdepth4 = 0;
   int cnodes = 0, cdepth = 0, cdepth4 = 0;
+  int tnodes4 = 0, snodes4 = 0, cnodes4 = 0;   // 4-wide inner nodes
   float tsah = 0.f, ssah = 0.f, csah = 0.f;   // SAH cost of each tree over its root's surface
   void free_built() {
     for (void *p : owned) dfree(p);
@@ -576,7 +577,13 @@ static int make_trace_params(const Visualization_ispc *vis, float global_eps, Tr
     if (!M->committed) return fail("model used before gxy_model_commit");
     P.has_model = (M->d.ntris > 0 || M->d.nsph > 0 || M->d.ncurve > 0) ? 1 : 0;
     P.model = M->d;
-    P.model.wide = (G.bvh_width == 4 && (M->d.ntris == 0 || M->d.tnodes4) && (M->d.nsph == 0 || M->d.snodes4)) ? 1 : 0;
+    // the 4-wide walk's bounds: at most three stack entries per level, byte
+    // offsets of nodes (128 B) and primitives (at most 36 B) in 32 bits
+    const int np = std::max(std::max(M->d.ntris, M->d.nsph), M->d.ncurve);
+    const int nn = std::max(std::max(M->tnodes4, M->snodes4), M->cnodes4);
+    const bool fits = wide_walk_fits(M->d.depth4, nn, np) && (M->d.ntris == 0 || M->d.tnodes4) &&
+                      (M->d.nsph == 0 || M->d.snodes4) && (M->d.ncurve == 0 || M->d.cnodes4);
+    P.model.wide = !fits ? 0 : G.bvh_width == 4 ? 1 : 2;
     P.hit_geom = M->hit_geom;
     P.hit_prim = M->hit_prim;
   }
@@ -1592,6 +1599,7 @@ GXY_EXPORT int gxy_model_commit(void *model) {
     if (validate_bvh4(B.nodes4, B.nnodes4, (int)ntri, "triangle") != 0) return -1;
     M->d.tnodes4 = B.nodes4;
     M->tdepth4 = B.depth4;
+    M->tnodes4 = B.nnodes4;
     M->tsah = B.sah;
   }
   if (nsph > 0) {
@@ -1638,6 +1646,7 @@ GXY_EXPORT int gxy_model_commit(void *model) {
     if (validate_bvh4(B.nodes4, B.nnodes4, (int)nsph, "sphere") != 0) return -1;
     M->d.snodes4 = B.nodes4;
     M->sdepth4 = B.depth4;
+    M->snodes4 = B.nnodes4;
     M->ssah = B.sah;
   }
   if (ncur > 0) {
@@ -1704,6 +1713,7 @@ GXY_EXPORT int gxy_model_commit(void *model) {
     if (validate_bvh4(B.nodes4, B.nnodes4, (int)ncur, "curve") != 0) return -1;
     M->d.cnodes4 = B.nodes4;
     M->cdepth4 = B.depth4;
+    M->cnodes4 = B.nnodes4;
     M->csah = B.sah;
     HIPCHK(hipStreamSynchronize(s));
   }
@@ -3095,7 +3105,7 @@ static int batch_dataset_params(BatchObj *B, const Visualization_ispc *vis, floa
   depth = 0;
   if (geometry) {
     ModelObj *M = lookup<ModelObj>(G.models, vis->model);
-    depth = M ? (P.model.wide ? M->d.depth4 : std::max(M->tdepth, M->sdepth)) : 64;
+    depth = M ? (P.model.wide == 1 ? M->d.depth4 : std::max(M->tdepth, M->sdepth)) : 64;
   }
   return 0;
 }

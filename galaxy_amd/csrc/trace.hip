@@ -11,89 +11,9 @@
 // comments at each stage); geometry follows Embree/OSPRay closest-hit and
 // postIntersect rules with the deterministic tie rule (equal t -> lowest
 // geomID, then primID).
-#include "trace_dev.h"
+#include "trace_kernel.h"
 
 namespace gxy {
-
-// A per-item count added to *ctr: the wave's total, one 64-bit atomic per wave
-// (every lane of the wave calls it)
-__device__ __forceinline__ void wave_add_count(unsigned long long v, unsigned long long *ctr) {
-  v = wave_sum_u64(v);
-  if ((threadIdx.x & 63) == 0 && v) atomicAdd(ctr, v);
-}
-
-// WPE > 0 asks the compiler for at least WPE waves per SIMD (fewer VGPRs);
-// the autotuner picks the variant.
-// SM = 1 when every volume is small (32-bit voxel offsets), -1 otherwise.
-// STK > 0: the BVH traversal stack holds STK entries per work-item in LDS
-// (instead of 64 in private memory).
-// W: BVH walked by geometry variants (2 binary, 4 four-wide, 0 per model).
-// MI: isovalues per volume the iso test is unrolled for (1 when no volume
-// has more than one, fewer scalar branches per sample).
-// BS: work-items per workgroup (64, 128 or 256).  A workgroup's slots are
-// refilled only as a whole, so smaller workgroups let a SIMD take new rays as
-// soon as one wave's rays are done, at the price of staging the transfer
-// function tables once per wave.
-// Workgroups reach the eight XCDs (one L2 each) round robin; this renumbering
-// hands each XCD runs of C consecutive workgroups' rays instead (neighbouring
-// camera tiles read the same bricks), the runs still dealt round robin so the
-// XCDs' shares of the image stay alike.  C = 1 is the dispatch order itself;
-// the workgroups past the last whole round of 8*C keep their own numbers.
-template <int C>
-__device__ __forceinline__ int xcd_block() {
-  const int b = blockIdx.x;
-  if (C <= 1) return b;
-  const int full = (int)gridDim.x / (8 * C) * (8 * C);
-  if (b >= full) return b;
-  const int x = b & 7, j = b >> 3;
-  return ((j / C) * 8 + x) * C + j % C;
-}
-
-template <int NV, bool GEOM, int WPE, int SM, int STK = 0, int W = 0, int MI = GXY_MAX_ISO, int BS = GXY_BLOCK>
-__global__ __launch_bounds__(BS) __attribute__((amdgpu_waves_per_eu(WPE > 0 ? WPE : 1, 8)))
-void k_trace(TraceParams P, RayList_ispc R, int n) {
-  constexpr int NVS = NV > 0 ? NV : 1;
-  __shared__ float s_col[NVS][3 * GXY_TF_MAX];
-  __shared__ float s_op[NVS][GXY_TF_MAX];
-  // a launch queued before its list's size was known covers the capacity:
-  // workgroups past the size leave at once (before staging the TF tables)
-  const int blk = xcd_block<(NV > 0 && !GEOM && STK == 0) ? 8 : 1>();
-  if (P.dn) {
-    n = min(n, *P.dn * P.dn_mul);
-    if (blk * BS >= n) return;
-  }
-#pragma unroll
-  for (int v = 0; v < NV; v++) {
-    for (int k = threadIdx.x; k < 3 * P.vv[v].tf.nc; k += BS) s_col[v][k] = P.vv[v].tf.col[k];
-    for (int k = threadIdx.x; k < P.vv[v].tf.no; k += BS) s_op[v][k] = P.vv[v].tf.op[k];
-  }
-  if (NV > 0) __syncthreads();
-
-  const int i = blk * BS + threadIdx.x;
-  unsigned long long nsamp = 0;
-  if (STK > 0) {
-    __shared__ int s_stack[STK > 0 ? STK : 1][BS];
-    LdsStack<(STK > 0 ? STK : 1)> stack;
-    stack.base = &s_stack[0][threadIdx.x];
-    stack.stride = BS;
-    if (i < n) nsamp = trace_one<NV, GEOM, LdsStack<(STK > 0 ? STK : 1)>, SM, W, MI>(P, R, i, s_col, s_op, stack);
-  } else if (NV > 0 && !GEOM) {
-    // volumes only: a wave whose rays are all primary, or all not, takes the
-    // march compiled for that kind (lists of one kind are the usual case)
-    PrivStack<GXY_BVH_STACK> stack;
-    if (i < n) {
-      const unsigned long long pm = __builtin_amdgcn_ballot_w64(gptr(R.type)[i] == RAY_PRIMARY);
-      const unsigned long long am = __builtin_amdgcn_ballot_w64(true);
-      if (pm == am) nsamp = trace_one<NV, GEOM, PrivStack<GXY_BVH_STACK>, SM, W, MI, 1>(P, R, i, s_col, s_op, stack);
-      else if (pm == 0) nsamp = trace_one<NV, GEOM, PrivStack<GXY_BVH_STACK>, SM, W, MI, 2>(P, R, i, s_col, s_op, stack);
-      else nsamp = trace_one<NV, GEOM, PrivStack<GXY_BVH_STACK>, SM, W, MI>(P, R, i, s_col, s_op, stack);
-    }
-  } else {
-    PrivStack<GXY_BVH_STACK> stack;
-    if (i < n) nsamp = trace_one<NV, GEOM, PrivStack<GXY_BVH_STACK>, SM, W, MI>(P, R, i, s_col, s_op, stack);
-  }
-  if (P.sample_count) wave_add_count(nsamp, P.sample_count);
-}
 
 // ------------------------------------------------------------- persistent-lane march
 // The same per-ray computation as k_trace (volumes, no geometry), organised so
@@ -391,17 +311,17 @@ static void launch_trace_sm(const TraceParams &P, const RayList_ispc &R, int n, 
   const bool one_iso = P.vv[0].nIso <= 1;
   if (one_iso && wpe == 6 && bs != 256) {
     dim3 gs((n + bs - 1) / bs), bb(bs);
-    if (bs == 64) hipLaunchKernelGGL((k_trace<1, false, 6, SM, 0, 0, 1, 64>), gs, bb, 0, s, P, R, n);
-    else hipLaunchKernelGGL((k_trace<1, false, 6, SM, 0, 0, 1, 128>), gs, bb, 0, s, P, R, n);
+    if (bs == 64) hipLaunchKernelGGL((k_trace<1, false, 6, SM, 1, 64>), gs, bb, 0, s, P, R, n);
+    else hipLaunchKernelGGL((k_trace<1, false, 6, SM, 1, 128>), gs, bb, 0, s, P, R, n);
     return;
   }
-  if (wpe == 5 && one_iso) hipLaunchKernelGGL((k_trace<1, false, 5, SM, 0, 0, 1>), g, b, 0, s, P, R, n);
+  if (wpe == 5 && one_iso) hipLaunchKernelGGL((k_trace<1, false, 5, SM, 1>), g, b, 0, s, P, R, n);
   else if (wpe == 5) hipLaunchKernelGGL((k_trace<1, false, 5, SM>), g, b, 0, s, P, R, n);
-  else if (wpe == 6 && one_iso) hipLaunchKernelGGL((k_trace<1, false, 6, SM, 0, 0, 1>), g, b, 0, s, P, R, n);
-  else if (wpe == 7 && one_iso) hipLaunchKernelGGL((k_trace<1, false, 7, SM, 0, 0, 1>), g, b, 0, s, P, R, n);
-  else if (wpe == 8 && one_iso) hipLaunchKernelGGL((k_trace<1, false, 8, SM, 0, 0, 1>), g, b, 0, s, P, R, n);
+  else if (wpe == 6 && one_iso) hipLaunchKernelGGL((k_trace<1, false, 6, SM, 1>), g, b, 0, s, P, R, n);
+  else if (wpe == 7 && one_iso) hipLaunchKernelGGL((k_trace<1, false, 7, SM, 1>), g, b, 0, s, P, R, n);
+  else if (wpe == 8 && one_iso) hipLaunchKernelGGL((k_trace<1, false, 8, SM, 1>), g, b, 0, s, P, R, n);
   else if (wpe >= 6) hipLaunchKernelGGL((k_trace<1, false, 6, SM>), g, b, 0, s, P, R, n);
-  else if (one_iso) hipLaunchKernelGGL((k_trace<1, false, 0, SM, 0, 0, 1>), g, b, 0, s, P, R, n);
+  else if (one_iso) hipLaunchKernelGGL((k_trace<1, false, 0, SM, 1>), g, b, 0, s, P, R, n);
   else hipLaunchKernelGGL((k_trace<1, false, 0, SM>), g, b, 0, s, P, R, n);
 }
 static void launch_trace_bricked(const TraceParams &P, const RayList_ispc &R, int n, int wpe, int bs, int sm, dim3 g,
@@ -427,26 +347,13 @@ static hipError_t launch_trace_nv(const TraceParams &P, const RayList_ispc &R, i
   dim3 g((n + GXY_BLOCK - 1) / GXY_BLOCK), b(GXY_BLOCK);
   bool small = true;
   for (int v = 0; v < NV; v++) small = small && P.vv[v].vol.small;
-  // an LDS stack only when it holds the deepest path of the model
-  if (NV == 0 && P.has_model && stack > 0 && (P.model.wide ? P.model.depth4 : P.model.depth) + 2 > stack) stack = 0;
-  const bool wide = P.model.wide != 0;
-  if (NV == 0 && P.has_model && P.model.ncurve > 0) {
-    // path lines: the variants that trace curve pieces too (private stack)
-    if (wide) hipLaunchKernelGGL((k_trace<0, true, 0, -1, 0, 20>), g, b, 0, s, P, R, n);
-    else if (gwaves == 8) hipLaunchKernelGGL((k_trace<0, true, 8, -1, 0, 18>), g, b, 0, s, P, R, n);
-    else hipLaunchKernelGGL((k_trace<0, true, 0, -1, 0, 18>), g, b, 0, s, P, R, n);
-  } else if (NV == 0 && P.has_model && wide) {
-    if (stack == 16) hipLaunchKernelGGL((k_trace<0, true, 0, -1, 16, 4>), g, b, 0, s, P, R, n);
-    else if (stack == 24) hipLaunchKernelGGL((k_trace<0, true, 0, -1, 24, 4>), g, b, 0, s, P, R, n);
-    else if (stack == 32) hipLaunchKernelGGL((k_trace<0, true, 0, -1, 32, 4>), g, b, 0, s, P, R, n);
-    else hipLaunchKernelGGL((k_trace<0, true, 0, -1, 0, 4>), g, b, 0, s, P, R, n);
-  } else if (NV == 0 && P.has_model) {
-    if (stack == 16) hipLaunchKernelGGL((k_trace<0, true, 0, -1, 16, 2>), g, b, 0, s, P, R, n);
-    else if (stack == 24) hipLaunchKernelGGL((k_trace<0, true, 0, -1, 24, 2>), g, b, 0, s, P, R, n);
-    else if (stack == 32) hipLaunchKernelGGL((k_trace<0, true, 0, -1, 32, 2>), g, b, 0, s, P, R, n);
-    else if (gwaves == 8) hipLaunchKernelGGL((k_trace<0, true, 8, -1, 0, 2>), g, b, 0, s, P, R, n);
-    else hipLaunchKernelGGL((k_trace<0, true, 0, -1, 0, 2>), g, b, 0, s, P, R, n);
-  } else if (P.has_model) hipLaunchKernelGGL((k_trace<NV, true, 0, -1>), g, b, 0, s, P, R, n);
+  if (NV == 0 && P.has_model) return launch_trace_geom(P, R, n, stack, gwaves, s);
+  if (P.has_model) {
+    // the walk as launch_trace_geom chooses it
+    TraceParams Q = P;
+    if (P.model.wide == 2 && (stack != 0 || gwaves != 0)) Q.model.wide = 0;
+    hipLaunchKernelGGL((k_trace<NV, true, 0, -1>), g, b, 0, s, Q, R, n);
+  }
   else if (NV == 1 && P.vv[0].vol.brick) launch_trace_bricked(P, R, n, wpe, trace_block_size(P, wpe, bs), sm_of(P.vv[0].vol), g, b, s);
   else if (small && wpe == 5) hipLaunchKernelGGL((k_trace<NV, false, 5, 1>), g, b, 0, s, P, R, n);
   else if (small && wpe >= 6) hipLaunchKernelGGL((k_trace<NV, false, 6, 1>), g, b, 0, s, P, R, n);

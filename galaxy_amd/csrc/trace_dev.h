@@ -22,8 +22,8 @@ struct GeoHit {
 
 // ------------------------------------------------------------- geometry
 struct WRay {
-  f3 org, dir;
-  int kx, ky, kz;
+  f3 org;
+  int k;   // axes kx, ky, kz in bits 0-1, 2-3, 4-5 (one register through the walk)
   float Sx, Sy, Sz;
 };
 
@@ -32,7 +32,6 @@ __device__ __forceinline__ float comp3(f3 a, int k) { return k == 0 ? a.x : (k =
 __device__ __forceinline__ WRay make_wray(f3 o, f3 d) {
   WRay r;
   r.org = o;
-  r.dir = d;
   float ax = fabsf(d.x), ay = fabsf(d.y), az = fabsf(d.z);
   int kz = 0;
   float m = ax;
@@ -41,7 +40,7 @@ __device__ __forceinline__ WRay make_wray(f3 o, f3 d) {
   int kx = kz + 1 == 3 ? 0 : kz + 1;
   int ky = kx + 1 == 3 ? 0 : kx + 1;
   if (comp3(d, kz) < 0.f) { int t = kx; kx = ky; ky = t; }
-  r.kx = kx; r.ky = ky; r.kz = kz;
+  r.k = kx | ky << 2 | kz << 4;
   float dz = comp3(d, kz);
   r.Sx = comp3(d, kx) / dz;
   r.Sy = comp3(d, ky) / dz;
@@ -53,10 +52,11 @@ __device__ __forceinline__ WRay make_wray(f3 o, f3 d) {
 __device__ __forceinline__ bool tri_hit(const WRay &r, f3 p0, f3 p1, f3 p2, float t0, float tfar, float &t,
                                         float &u, float &v) {
   f3 A = sub3(p0, r.org), B = sub3(p1, r.org), Cc = sub3(p2, r.org);
-  float Az_ = comp3(A, r.kz), Bz_ = comp3(B, r.kz), Cz_ = comp3(Cc, r.kz);
-  float Ax = comp3(A, r.kx) - r.Sx * Az_, Ay = comp3(A, r.ky) - r.Sy * Az_;
-  float Bx = comp3(B, r.kx) - r.Sx * Bz_, By = comp3(B, r.ky) - r.Sy * Bz_;
-  float Cx = comp3(Cc, r.kx) - r.Sx * Cz_, Cy = comp3(Cc, r.ky) - r.Sy * Cz_;
+  const int kx = r.k & 3, ky = r.k >> 2 & 3, kz = r.k >> 4;
+  float Az_ = comp3(A, kz), Bz_ = comp3(B, kz), Cz_ = comp3(Cc, kz);
+  float Ax = comp3(A, kx) - r.Sx * Az_, Ay = comp3(A, ky) - r.Sy * Az_;
+  float Bx = comp3(B, kx) - r.Sx * Bz_, By = comp3(B, ky) - r.Sy * Bz_;
+  float Cx = comp3(Cc, kx) - r.Sx * Cz_, Cy = comp3(Cc, ky) - r.Sy * Cz_;
   float U = Cx * By - Cy * Bx;
   float V = Ax * Cy - Ay * Cx;
   float W = Bx * Ay - By * Ax;
@@ -179,29 +179,49 @@ __device__ __forceinline__ bool better(float t, int g, int p, const GeoHit &h) {
   return false;
 }
 
-#define GXY_BVH_STACK 64
 #define GXY_SENTINEL 0x7fffffff
 
-// Per-lane traversal stacks.  PrivStack keeps the entries in private memory
-// (scratch, cached per lane); LdsStack keeps them in LDS with entry k of a
-// lane at base[k * stride] (stride = lanes of the workgroup, so lanes at the
-// same depth touch consecutive words).  DEPTH entries; a model whose tree is
-// deeper than DEPTH - 2 must not be traced with it (checked on the host).
-template <int SD>
-struct PrivStack {
-  static constexpr int DEPTH = SD;
-  int s[SD];
-  __device__ __forceinline__ void put(int k, int v) { s[k] = v; }
-  __device__ __forceinline__ int get(int k) const { return s[k]; }
-};
-
-template <int SD>
-struct LdsStack {
-  static constexpr int DEPTH = SD;
+// Per-lane traversal stack: the first NL entries in LDS (entry k of a lane at
+// base[k * BS], so a wave's accesses are free of bank conflicts whatever the
+// lanes' depths), the rest in private memory.  Deep enough for every tree, while
+// the entries that a walk touches most of the time cost an LDS access and not a
+// trip to the vector cache (icosphere walks pop 45 entries per wave, nearly all
+// of them within the first 16).
+#define GXY_LDS_STACK 16
+#define GXY_STACK_OVER 64   // (wide_walk_fits counts on the sum of the two)
+struct NoStack {};
+template <int NL, int BS>
+struct HybStack {
+  static constexpr int OVER = GXY_STACK_OVER;
+  static constexpr int DEPTH = NL + OVER;
   int *base;
-  int stride;
-  __device__ __forceinline__ void put(int k, int v) { base[k * stride] = v; }
-  __device__ __forceinline__ int get(int k) const { return base[k * stride]; }
+  int over[OVER];
+  __device__ __forceinline__ void put(int k, int v) {
+    if (k < NL) base[k * BS] = v;
+    else over[k - NL] = v;
+  }
+  __device__ __forceinline__ int get(int k) const { return k < NL ? base[k * BS] : over[k - NL]; }
+  __device__ __forceinline__ int pop(int &sp) const { return get(--sp); }
+  // pushes the codes whose flag is set.  While every lane of the wave has four
+  // LDS entries free, each code is written at the top and kept by moving it.
+  __device__ __forceinline__ void push4(int &sp, int c0, bool k0, int c1, bool k1, int c2, bool k2, int c3, bool k3) {
+    if (__builtin_amdgcn_ballot_w64(sp > NL - 4) == 0) {
+      int *p = base + sp * BS;
+      *p = c0;
+      p += k0 ? BS : 0;
+      *p = c1;
+      p += k1 ? BS : 0;
+      *p = c2;
+      p += k2 ? BS : 0;
+      *p = c3;
+      sp += (k0 ? 1 : 0) + (k1 ? 1 : 0) + (k2 ? 1 : 0) + (k3 ? 1 : 0);
+    } else {
+      if (k0) put(sp++, c0);
+      if (k1) put(sp++, c1);
+      if (k2) put(sp++, c2);
+      if (k3) put(sp++, c3);
+    }
+  }
 };
 
 // Slab test of one child box against [t0, tmax] with a few ulps of slack so
@@ -258,108 +278,94 @@ __device__ __forceinline__ void bvh_walk(const BVHNode *nodes, f3 o, f3 inv, flo
   }
 }
 
-// Nearest-first walk of a 4-wide BVH.  At a node, the children's boxes are
-// tested against [t0, current hit t]; leaf children that are hit are
-// intersected at once (the LBVH leaves hold one primitive), then the walk
-// descends into the nearest inner child that is still hit and pushes one
-// entry (node << 4 | mask of the other hit inner children), re-tested against
-// the then-current hit t when popped, so the stack holds at most one entry per
-// level (depth4 entries).
+// Nearest-first walk of a 4-wide BVH.  A node visit tests the four child boxes
+// and takes the nearest hit child next; the other hit children, inner nodes and
+// leaves alike, go on the stack, each an entry of its own (never more than
+// three per level: the launcher takes this walk only when 3 * depth4 + 2
+// entries fit).  What bounds it is VALU issue (a wave's lanes are at different
+// nodes most of the time), so a visit is kept short and without branches:
+// - a box plane costs one FMA, p * (1/d) - o * (1/d).  Its rounding error is
+//   at most 2^-23 |o/d| + 2^-23 |t|, so the near planes are moved towards the
+//   origin and the far planes away from it by 2^-21 |o/d| and the far planes
+//   scaled by 1 + 1.2e-6: a box is only ever entered needlessly, never missed.
+//   An axis whose direction underflows (1/d infinite) gives NaN planes, which
+//   max and min skip;
+// - the near and far planes of an axis are loaded from the lo or hi row by a
+//   per-ray byte offset instead of being selected after the load;
+// - every child is written to the top of the stack and the top moves only for
+//   the children kept, so no lane branches to push.
 template <class Stack, class LeafFn>
 __device__ __forceinline__ void bvh4_walk(const BVH4Node *nodes, f3 o, f3 inv, float t0, const GeoHit &h,
-                                          Stack &stack, LeafFn &&leaf, bool any, int dlim) {
+                                          Stack &stack, LeafFn &&leaf, bool any) {
+  // (a ray with a NaN or infinite coordinate hits nothing)
+  if (!(fabsf(o.x) < 3.4e38f && fabsf(o.y) < 3.4e38f && fabsf(o.z) < 3.4e38f) || inv.x != inv.x || inv.y != inv.y ||
+      inv.z != inv.z)
+    return;
+  constexpr float FS = 1.0000012f, PAD = 4.76837158e-7f;
+  const float ox = o.x * inv.x, oy = o.y * inv.y, oz = o.z * inv.z;
+  const float px = PAD * fabsf(ox), py = PAD * fabsf(oy), pz = PAD * fabsf(oz);
+  const float nx = -ox - px, ny = -oy - py, nz = -oz - pz;
+  const float fx = px - ox * FS, fy = py - oy * FS, fz = pz - oz * FS;
+  const f3 invf = mk3(inv.x * FS, inv.y * FS, inv.z * FS);
+  const unsigned bx = inv.x < 0.f ? 48u : 0u, by = inv.y < 0.f ? 64u : 16u, bz = inv.z < 0.f ? 80u : 32u;
+  const char *nb = (const char *)gptr(nodes);
   int sp = 0;
-  int cur = 0, mask = 0xF;
-  const BVH4Node *gn = gptr(nodes);
-  for (;;) {
-    const float4 *np = (const float4 *)(gn + cur);
-    const float4 lx = np[0], ly = np[1], lz = np[2], hx = np[3], hy = np[4], hz = np[5];
-    const int4 ch = ((const int4 *)np)[6];
-    const float lox[4] = {lx.x, lx.y, lx.z, lx.w}, loy[4] = {ly.x, ly.y, ly.z, ly.w}, loz[4] = {lz.x, lz.y, lz.z, lz.w};
-    const float hix[4] = {hx.x, hx.y, hx.z, hx.w}, hiy[4] = {hy.x, hy.y, hy.z, hy.w}, hiz[4] = {hz.x, hz.y, hz.z, hz.w};
-    const int cc[4] = {ch.x, ch.y, ch.z, ch.w};
-    float te[4];
-    int inner = 0, leaves = 0;
+  stack.put(sp++, GXY_SENTINEL);
+  int cur = 0;
+  while (cur != GXY_SENTINEL) {
+    bool pop = true;
+    if (cur >= 0) {
+      const unsigned w = (unsigned)cur << 7;   // under 2^25 nodes (checked by the launcher)
+      // (rows at 0 16 32 | 48 64 80: an axis's two rows differ by the bits 48, 80, 112)
+      const unsigned wx = w | bx, wy = w | by, wz = w | bz;
+      const float4 nX = *(const float4 *)(nb + wx), fX = *(const float4 *)(nb + (wx ^ 48u));
+      const float4 nY = *(const float4 *)(nb + wy), fY = *(const float4 *)(nb + (wy ^ 80u));
+      const float4 nZ = *(const float4 *)(nb + wz), fZ = *(const float4 *)(nb + (wz ^ 112u));
+      const int4 ch = *(const int4 *)(nb + (w + 96u));
+      const float hts = __builtin_fmaf(h.t, 1.0000005f, 1e-30f);
+      const float inf = __builtin_inff();
+      float t[4];
+      bool hit[4];
+      const float anx[4] = {nX.x, nX.y, nX.z, nX.w}, afx[4] = {fX.x, fX.y, fX.z, fX.w};
+      const float any_[4] = {nY.x, nY.y, nY.z, nY.w}, afy[4] = {fY.x, fY.y, fY.z, fY.w};
+      const float anz[4] = {nZ.x, nZ.y, nZ.z, nZ.w}, afz[4] = {fZ.x, fZ.y, fZ.z, fZ.w};
 #pragma unroll
-    for (int k = 0; k < 4; k++) {
-      te[k] = 0.f;
-      if ((mask >> k) & 1) {
-        const float lo[3] = {lox[k], loy[k], loz[k]}, hi[3] = {hix[k], hiy[k], hiz[k]};
-        if (child_hit(lo, hi, o, inv, t0, h.t, te[k])) {
-          if (cc[k] >= 0) inner |= 1 << k;
-          else leaves |= 1 << k;
-        }
+      for (int k = 0; k < 4; k++) {
+        const float tn = __builtin_fmaxf(__builtin_fmaxf(__builtin_fmaf(anx[k], inv.x, nx), __builtin_fmaf(any_[k], inv.y, ny)),
+                                         __builtin_fmaxf(__builtin_fmaf(anz[k], inv.z, nz), t0));
+        const float tf = __builtin_fminf(__builtin_fminf(__builtin_fmaf(afx[k], invf.x, fx), __builtin_fmaf(afy[k], invf.y, fy)),
+                                         __builtin_fminf(__builtin_fmaf(afz[k], invf.z, fz), hts));
+        hit[k] = tn <= tf;
+        t[k] = hit[k] ? tn : inf;
       }
-    }
-    // the hit leaf children in slot order, through one copy of the leaf code
-    // (a wave runs it as often as its lanes' largest leaf count)
-    while (leaves) {
-      const int k = __builtin_ctz(leaves);
-      leaves &= leaves - 1;
-      int c = cc[0];
-#pragma unroll
-      for (int q = 1; q < 4; q++) c = (q == k) ? cc[q] : c;
-      const int code = ~c;
+      const float tm = __builtin_fminf(__builtin_fminf(t[0], t[1]), __builtin_fminf(t[2], t[3]));
+      const int c0 = ch.x, c1 = ch.y, c2 = ch.z, c3 = ch.w;
+      // (keeps the load of the codes beside those of the planes)
+      asm volatile("" ::"v"(c0), "v"(c1), "v"(c2), "v"(c3));
+      if (tm < inf) {
+        cur = t[2] == tm ? c2 : c3;
+        cur = t[1] == tm ? c1 : cur;
+        cur = t[0] == tm ? c0 : cur;
+        stack.push4(sp, c0, hit[0] && cur != c0, c1, hit[1] && cur != c1, c2, hit[2] && cur != c2, c3,
+                    hit[3] && cur != c3);
+        pop = false;
+      }
+    } else {
+      const int code = ~cur;
       leaf(code >> 4, (code & 15) + 1);
       if (any && h.geom >= 0) return;
     }
-    // the nearest inner child whose box still starts before the current hit
-    int kn = -1;
-    float tn = 0.f;
-#pragma unroll
-    for (int k = 0; k < 4; k++)
-      if (((inner >> k) & 1) && te[k] <= h.t * 1.0000005f + 1e-30f && (kn < 0 || te[k] < tn)) {
-        kn = k;
-        tn = te[k];
-      }
-    if (kn >= 0) {
-      int rest = inner & ~(1 << kn);
-      if (rest && sp <= dlim) {
-        // the other children still hit, each its own entry, the nearest on top
-#pragma unroll
-        for (int k = 0; k < 4; k++)
-          if (((rest >> k) & 1) && !(te[k] <= h.t * 1.0000005f + 1e-30f)) rest &= ~(1 << k);
-        while (rest) {
-          int kf = __builtin_ctz(rest);
-          float tf = te[0];
-#pragma unroll
-          for (int k = 1; k < 4; k++) tf = (k == kf) ? te[k] : tf;
-#pragma unroll
-          for (int k = 0; k < 4; k++)
-            if (((rest >> k) & 1) && te[k] > tf) {
-              kf = k;
-              tf = te[k];
-            }
-          rest &= ~(1 << kf);
-          int c2 = cc[0];
-#pragma unroll
-          for (int k = 1; k < 4; k++) c2 = (k == kf) ? cc[k] : c2;
-          stack.put(sp++, c2 << 4);
-        }
-      } else if (rest && sp < Stack::DEPTH) {
-        if ((rest & (rest - 1)) == 0) {
-          // one other child: its own node, whole (mask 0)
-          const int k2 = __builtin_ctz(rest);
-          int c2 = cc[0];
-#pragma unroll
-          for (int k = 1; k < 4; k++) c2 = (k == k2) ? cc[k] : c2;
-          stack.put(sp++, c2 << 4);
-        } else {
-          stack.put(sp++, (cur << 4) | rest);
-        }
-      }
-      int c = cc[0];
-#pragma unroll
-      for (int k = 1; k < 4; k++) c = (k == kn) ? cc[k] : c;
-      cur = c;
-      mask = 0xF;
-      continue;
-    }
-    if (sp == 0) return;
-    const int e = stack.get(--sp);
-    cur = e >> 4;
-    mask = (e & 15) ? (e & 15) : 0xF;
+    if (pop) cur = stack.pop(sp);
   }
+}
+
+// Element k of a primitive array of `per` words each: a uniform base and a
+// 32-bit byte offset where every array of the model spans under 4 GiB (S; the
+// 4-wide walks, checked by the launcher), a 64-bit address otherwise.
+template <bool S, class T>
+__device__ __forceinline__ const T *prim_at(const T *base, int k, int per) {
+  if (S) return (const T *)((const char *)gptr(base) + (size_t)((unsigned)k * (unsigned)(per * sizeof(T))));
+  return gptr(base) + (int64_t)per * k;
 }
 
 // W: 2 or 4, the tree width the walks use; 0, either (chosen per call from
@@ -379,39 +385,37 @@ __device__ __forceinline__ void model_trace(const DModel &M, f3 org, f3 dir, flo
   if (tfar < t0) return;
   constexpr int TW = W & 15;
   f3 inv = mk3(1.0f / dir.x, 1.0f / dir.y, 1.0f / dir.z);
-  // 4-wide walks: stack depth up to which other hit children get entries of their own
-  const int dlim = Stack::DEPTH - M.depth4 - 3;
   if (M.ntris > 0) {
     WRay wr = make_wray(org, dir);
     auto tleaf = [&](int start, int count) {
       for (int k = start; k < start + count; k++) {
-        const float *p = gptr(M.tverts) + 9 * (int64_t)k;
+        const float *p = prim_at<TW == 4>(M.tverts, k, 9);
         f3 p0 = mk3(p[0], p[1], p[2]), p1 = mk3(p[3], p[4], p[5]), p2 = mk3(p[6], p[7], p[8]);
         float t, u, v;
         if (tri_hit(wr, p0, p1, p2, t0, h.t, t, u, v)) {
-          int g = gptr(M.tgeom)[k], pr = gptr(M.tprim)[k];
+          int g = *prim_at<TW == 4>(M.tgeom, k, 1), pr = *prim_at<TW == 4>(M.tprim, k, 1);
           if (h.geom < 0 || better(t, g, pr, h)) { h.t = t; h.geom = g; h.prim = pr; h.u = u; h.v = v; }
         }
       }
     };
-    if (TW == 4 || (TW == 0 && M.wide)) bvh4_walk(M.tnodes4, org, inv, t0, h, stack, tleaf, any, dlim);
+    if (TW == 4 || (TW == 0 && M.wide)) bvh4_walk(M.tnodes4, org, inv, t0, h, stack, tleaf, any);
     else bvh_walk(M.tnodes, org, inv, t0, h, stack, tleaf, any);
   }
   if (any && h.geom >= 0) return;
   if (M.nsph > 0) {
     auto sleaf = [&](int start, int count) {
       for (int k = start; k < start + count; k++) {
-        const float *sc = gptr(M.scenter);
-        f3 c = mk3(sc[3 * k], sc[3 * k + 1], sc[3 * k + 2]);
+        const float *sc = prim_at<TW == 4>(M.scenter, k, 3);
+        f3 c = mk3(sc[0], sc[1], sc[2]);
         float lim = h.geom < 0 ? h.t : nextafterf(h.t, 3e38f);
         float t;
-        if (sphere_hit(c, gptr(M.sradius)[k], gptr(M.seps)[k], org, dir, t0, lim, t)) {
-          int g = gptr(M.sgeom)[k], pr = gptr(M.sprim)[k];
+        if (sphere_hit(c, *prim_at<TW == 4>(M.sradius, k, 1), *prim_at<TW == 4>(M.seps, k, 1), org, dir, t0, lim, t)) {
+          int g = *prim_at<TW == 4>(M.sgeom, k, 1), pr = *prim_at<TW == 4>(M.sprim, k, 1);
           if (h.geom < 0 || better(t, g, pr, h)) { h.t = t; h.geom = g; h.prim = pr; h.u = h.v = 0.f; }
         }
       }
     };
-    if (TW == 4 || (TW == 0 && M.wide)) bvh4_walk(M.snodes4, org, inv, t0, h, stack, sleaf, any, dlim);
+    if (TW == 4 || (TW == 0 && M.wide)) bvh4_walk(M.snodes4, org, inv, t0, h, stack, sleaf, any);
     else bvh_walk(M.snodes, org, inv, t0, h, stack, sleaf, any);
   }
   if (any && h.geom >= 0) return;
@@ -422,19 +426,19 @@ __device__ __forceinline__ void model_trace(const DModel &M, f3 org, f3 dir, flo
     // traversal order), h.v the piece (its sorted index) for the shading
     auto cleaf = [&](int start, int count) {
       for (int k = start; k < start + count; k++) {
-        const float *A = gptr(M.ca) + 4 * (int64_t)k, *B = gptr(M.cb) + 4 * (int64_t)k;
+        const float *A = prim_at<TW == 4>(M.ca, k, 4), *B = prim_at<TW == 4>(M.cb, k, 4);
         float lim = h.geom < 0 ? h.t : nextafterf(h.t, 3e38f);
         float t;
         if (roundcone_hit(mk3(A[0], A[1], A[2]), A[3], mk3(B[0], B[1], B[2]), B[3], org, dir, t0, lim, t)) {
-          const int g = gptr(M.cgeom)[k], pr = gptr(M.cprim)[k];
-          const float u0 = gptr(M.cu)[2 * (int64_t)k];
+          const int g = *prim_at<TW == 4>(M.cgeom, k, 1), pr = *prim_at<TW == 4>(M.cprim, k, 1);
+          const float u0 = *prim_at<TW == 4>(M.cu, k, 2);
           if (h.geom < 0 || better(t, g, pr, h) || (t == h.t && g == h.geom && pr == h.prim && u0 < h.u)) {
             h.t = t; h.geom = g; h.prim = pr; h.u = u0; h.v = __int_as_float(k);
           }
         }
       }
     };
-    if (TW == 4 || (TW == 0 && M.wide)) bvh4_walk(M.cnodes4, org, inv, t0, h, stack, cleaf, any, dlim);
+    if (TW == 4 || (TW == 0 && M.wide)) bvh4_walk(M.cnodes4, org, inv, t0, h, stack, cleaf, any);
     else bvh_walk(M.cnodes, org, inv, t0, h, stack, cleaf, any);
   }
 }
@@ -554,6 +558,71 @@ __device__ __forceinline__ void composite(float &cr, float &cg, float &cb, float
   ca = __builtin_fmaf(a, wo, ca);
 }
 
+// One ray of TraceRays_TraceRays (TraceRays.ispc:371-622) through geometry
+// without volumes: box clip, closest hit (any hit for occlusion rays), shading.
+// What the march would need is not carried through the walk, so that more
+// waves fit: the colour, which geometry leaves as it is, is read afterwards for
+// the opacity test and not written back, and the direction is read again for
+// the shading of a primary ray's hit.
+// The ray is the k-th after ray `first` (uniform over the wave): its fields lie at
+// a uniform address and a 32-bit offset, which keeps one register of addressing
+// live through the walk instead of a 64-bit address per field.
+__device__ __forceinline__ f3 ray_org(const RayList_ispc &R, int first, unsigned k) {
+  return mk3(gptr(R.ox + first)[k], gptr(R.oy + first)[k], gptr(R.oz + first)[k]);
+}
+__device__ __forceinline__ f3 ray_dir(const RayList_ispc &R, int first, unsigned k) {
+  f3 dir = mk3(gptr(R.dx + first)[k], gptr(R.dy + first)[k], gptr(R.dz + first)[k]);
+  if (dir.x == 0.f) dir.x = 1e-6f;
+  if (dir.y == 0.f) dir.y = 1e-6f;
+  if (dir.z == 0.f) dir.z = 1e-6f;
+  return dir;
+}
+template <class Stack, int W>
+__device__ __forceinline__ void trace_geom_one(const TraceParams &P, const RayList_ispc &R, const int first,
+                                               const unsigned k, Stack &stack) {
+  bool shade;
+  int miss;   // the term of a ray that hits nothing
+  GeoHit gh;
+  {
+    const f3 org = ray_org(R, first, k), dir = ray_dir(R, first, k);
+    shade = gptr(R.type + first)[k] == RAY_PRIMARY;
+    float t0 = gptr(R.t + first)[k];
+    const float tTimeout = gptr(R.tMax + first)[k];
+    // box clip (TraceRays.ispc:406-418)
+    float tEntry, tExit;
+    box_clip(org, dir, P.blo, P.bhi, tEntry, tExit);
+    if (tEntry > t0) t0 = tEntry;
+    const float tEnd = mnf(tTimeout, tExit);
+    miss = tEnd == tExit ? RAY_BOUNDARY : tEnd == tTimeout ? RAY_TIMEOUT : 0;
+    // LookForGeometryHit (TraceRays.ispc:108-141).  A shadow or AO ray needs
+    // only whether it is blocked (any hit terminates it with its own colour)
+    // when the host does not read its t (the rank loops; not
+    // TraceRays_TraceRays)
+    model_trace<Stack, W>(P.model, org, dir, t0, tEnd, gh, stack, P.occlusion && !shade);
+  }
+  if (P.hit_geom) { (P.hit_geom + first)[k] = gh.geom; (P.hit_prim + first)[k] = gh.prim; }
+  int term = opaque_of(gptr(R.r + first)[k], gptr(R.g + first)[k], gptr(R.b + first)[k], gptr(R.o + first)[k],
+                       P.opaque_alpha)
+                 ? RAY_OPAQUE
+                 : 0;
+  gptr(R.t + first)[k] = gh.t;
+  if (gh.geom >= 0) {
+    Hit hit;
+    hit.opacity = 0.f;
+    hit.normal = mk3(0.f, 0.f, 0.f);
+    hit.color = hit.normal;
+    if (shade) geom_shade<W>(P.model, gh, ray_org(R, first, k), ray_dir(R, first, k), hit);
+    term |= RAY_SURFACE;
+    if (hit.opacity > 0.999f) term |= RAY_OPAQUE;
+    gptr(R.sr + first)[k] = hit.color.x; gptr(R.sg + first)[k] = hit.color.y; gptr(R.sb + first)[k] = hit.color.z;
+    gptr(R.so + first)[k] = 1.0f;
+    gptr(R.nx + first)[k] = hit.normal.x; gptr(R.ny + first)[k] = hit.normal.y; gptr(R.nz + first)[k] = hit.normal.z;
+  } else {
+    term |= miss;
+  }
+  gptr(R.term + first)[k] = term;
+}
+
 // One ray of TraceRays_TraceRays (TraceRays.ispc:371-622): reads ray i of R,
 // writes its colour, t, term and surface fields back.  s_col / s_op hold the
 // NV transfer-function tables (LDS).  Returns the number of volume samples.
@@ -561,7 +630,7 @@ __device__ __forceinline__ void composite(float &cr, float &cg, float &cb, float
 // nIso must not exceed it).
 // SH: 1 when the caller has found every active lane's ray primary, 2 when it
 // has found none primary (the choice is then known to the compiler), 0 per lane.
-template <int NV, bool GEOM, class Stack, int SM = -1, int W = 0, int MI = GXY_MAX_ISO, int SH = 0>
+template <int NV, bool GEOM, int SM = -1, int MI = GXY_MAX_ISO, int SH = 0, class Stack>
 __device__ __forceinline__ unsigned trace_one(const TraceParams &P, const RayList_ispc &R, const int i,
                                               const float (*s_col)[3 * GXY_TF_MAX],
                                               const float (*s_op)[GXY_TF_MAX], Stack &stack) {
@@ -624,19 +693,16 @@ __device__ __forceinline__ unsigned trace_one(const TraceParams &P, const RayLis
         }
     }
 
-    // LookForGeometryHit (TraceRays.ispc:108-141)
-    if (GEOM) {
+    // LookForGeometryHit (TraceRays.ispc:108-141; geometry without volumes is
+    // traced by trace_geom_one)
+    if constexpr (GEOM) {
       GeoHit gh;
-      // a shadow or AO ray in a scene without volumes needs only whether it
-      // is blocked (any hit terminates it with its own colour) when the host
-      // does not read its t (the rank loops; not TraceRays_TraceRays)
-      const bool any = NV == 0 && P.occlusion && !shadeFlag;
-      model_trace<Stack, W>(P.model, org, dir, ray_t0, ray_t, gh, stack, any);
+      model_trace<Stack, 0>(P.model, org, dir, ray_t0, ray_t, gh, stack);
       if (P.hit_geom) { P.hit_geom[i] = gh.geom; P.hit_prim[i] = gh.prim; }
       if (gh.geom >= 0) {
         ray_t = gh.t;
         surface_hit = true;
-        if (shadeFlag) geom_shade<W>(P.model, gh, org, dir, hit);
+        if (shadeFlag) geom_shade<0>(P.model, gh, org, dir, hit);
       }
     }
 

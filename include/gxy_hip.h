@@ -200,10 +200,10 @@ float       gxy_get_opacity_threshold(void);
  * `refill` (1..64) of them are idle.  Results are identical for every setting;
  * galaxy_amd/autotune.py picks the fastest. */
 int         gxy_set_trace_config(int kind, int chunk, int refill);
-/* BVH traversal stack of geometry-only traces (no reference counterpart):
- * 0 = 64 entries per ray in private memory; 16 / 24 / 32 = that many entries
- * in LDS, used for models whose tree depth + 2 fits (others keep the private
- * stack).  Results are identical for every setting. */
+/* Binary BVH walk of geometry-only traces (no reference counterpart) with 16 /
+ * 24 / 32 traversal stack entries in LDS (deeper entries in private memory);
+ * 0 (default): the walk chosen by gxy_set_bvh_width.  Results are identical for
+ * every setting. */
 int         gxy_set_geometry_stack(int entries);
 int         gxy_get_geometry_stack(void);
 /* Occlusion rays (default 1): in the rank loops (gxy_render_frame,
@@ -214,19 +214,17 @@ int         gxy_get_geometry_stack(void);
  * 0: closest hit everywhere (same frames and counts). */
 int gxy_set_occlusion_rays(int on);
 int gxy_get_occlusion_rays(void);
-/* BVH traversed by geometry traces (no reference counterpart): 2 (default) =
- * the binary LBVH, 4 = the 4-wide trees every model commit also builds
- * (128-byte nodes, about half the depth).  Hits are identical either way.
- * The binary walk is faster on scenes of several objects and on path lines
- * (1.3-1.8x on MI355X), the 4-wide one by about 9% on one closed mesh. */
+/* BVH walked by geometry traces (no reference counterpart).  Every model commit
+ * builds a binary tree and its 4-wide collapse (128-byte nodes, about half the
+ * depth).  2 (default): the 4-wide walk, unless gxy_set_geometry_stack or
+ * gxy_set_geometry_waves asks for a binary one; 4: the 4-wide walk.  Trees
+ * beyond the 4-wide walk's bounds (26 levels, 2^25 nodes, 2^26 primitives) take
+ * the binary walk either way.  Hits are identical. */
 int         gxy_set_bvh_width(int width);
 int         gxy_get_bvh_width(void);
-/* Occupancy of the binary walks with the private stack, path lines included
- * (no reference counterpart): 0 (default) = the compiler's register
- * allocation (70 VGPRs, 7 waves per SIMD; 76 and 6 with path lines), 8 = 8
- * waves per SIMD (64 VGPRs, some spills; 4 % faster on the 11.8 M-triangle
- * nine-icosphere frame, 5 % on the path-line frame, 5 % slower on a
- * 20 K-triangle mesh).  Results are identical. */
+/* 8: the binary walk at 8 waves per SIMD (64 VGPRs, some spills), path lines
+ * included (no reference counterpart); 0 (default): the walk chosen by
+ * gxy_set_bvh_width at the occupancy it is tuned for.  Results are identical. */
 int         gxy_set_geometry_waves(int waves);
 int         gxy_get_geometry_waves(void);
 int         gxy_get_trace_config(int *kind, int *chunk, int *refill);
@@ -523,8 +521,8 @@ int   gxy_batch_add_list(void *batch, int ds, int mode, int n, const RayList_isp
 int   gxy_batch_set_list_seed(void *batch, int list, unsigned seed, const float lo[3], const float hi[3]);
 int   gxy_batch_remove_list(void *batch, int list);
 /* Launch configuration: chunk (rays per queue entry, 64..1024), stack (BVH traversal
- * stack: 0 = 64 entries in private memory, 16/24/32 = entries in LDS; must
- * exceed the deepest tree by 2), wpe (waves per SIMD requested: 0, 4, 5 or 6; with an
+ * stack: 0 = the 4-wide walk, 16/24/32 = the binary walk, or the 4-wide one with
+ * BVH width 4, with that many entries in LDS; must exceed the deepest tree by 2), wpe (waves per SIMD requested: 0, 4, 5 or 6; with an
  * LDS stack the fused kernel ignores 5 and 6, split mode applies it to the volume
  * kernel; in split mode the sampler kernel always asks for 8),
  * blocks_per_cu (persistent workgroups per compute unit, 1..16). */

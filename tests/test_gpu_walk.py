@@ -1,0 +1,131 @@
+"""The 4-wide BVH walk against the binary one: the same hits, t, colours and
+geometry / primitive IDs on every ray, the awkward ones included (axis-aligned
+and denormal directions, origins on box faces, infinite and NaN fields, empty
+intervals), over trees from one leaf to several thousand nodes."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from galaxy_amd import abi, scenes, workloads
+
+pytestmark = pytest.mark.gpu
+f32 = np.float32
+
+
+@pytest.fixture(scope="module")
+def hip():
+    from galaxy_amd import lib as glib
+    return glib.HipBackend()
+
+
+def _scene(kind):
+    rng = np.random.default_rng(3)
+    box = ((-0.5,) * 3, (1.5,) * 3)
+    sc = scenes.SceneDesc(local_box=box, global_box=box)
+    if kind.startswith("tris"):
+        # n triangles, axis-aligned ones (flat boxes) among them
+        n = int(kind[4:])
+        v = rng.uniform(0, 1, (n, 3, 3))
+        v[::2] = v[::2, :1] + rng.uniform(-0.2, 0.2, (len(v[::2]), 3, 3))
+        v[::3, :, 2] = v[::3, :1, 2]
+        sc.meshes = [scenes.MeshDesc(v.reshape(-1, 3).astype(f32), np.arange(3 * n, dtype=np.uint32).reshape(-1, 3))]
+    elif kind == "stacked":
+        # many equal triangles: ties in t, a tree without spatial order
+        v = np.tile(rng.uniform(0.2, 0.8, (4, 3, 3)), (300, 1, 1))
+        sc.meshes = [scenes.MeshDesc(v.reshape(-1, 3).astype(f32), np.arange(3600, dtype=np.uint32).reshape(-1, 3))]
+    elif kind == "blob_spheres":
+        sc.meshes = [scenes.blob_mesh(20000, 5)]
+        sc.spheres = [scenes.SpheresDesc(rng.uniform(0, 1, (3000, 3)).astype(f32), rng.uniform(0, 1, 3000).astype(f32),
+                                         0.005, 0.03, 0.0, 1.0)]
+    else:
+        sc.pathlines = workloads.pathlines(8, 8, 200, 24, 2)[0].pathlines
+    return sc
+
+
+def _rays():
+    rng = np.random.default_rng(8)
+    n = 6000
+    o = rng.uniform(-0.4, 1.4, (n, 3))
+    d = rng.normal(size=(n, 3))
+    d /= np.linalg.norm(d, axis=1, keepdims=True)
+    t0, tm = np.zeros(n), np.full(n, 1e30)
+    for a in range(3):                       # axis-aligned, both ways, and nearly so
+        k = slice(200 * a, 200 * a + 100)
+        d[k] = 0.0
+        d[k, a] = rng.choice([-1.0, 1.0], 100)
+        k = slice(200 * a + 100, 200 * a + 200)
+        d[k, a] = rng.choice([1e-30, -1e-30, 1e-40, -1e-44, -0.0, 1e-7], 100)
+    o[600:700] = np.round(o[600:700])        # origins on the scene's faces and corners
+    o[700:750] *= 1e4                        # far away, aimed back
+    d[700:750] = (0.5 - o[700:750]) / np.linalg.norm(0.5 - o[700:750], axis=1, keepdims=True)
+    tm[700:750] = 1e6
+    t0[750:800] = 0.3
+    tm[800:850] = 0.25
+    t0[850:860], tm[850:860] = 0.5, 0.2      # an empty interval
+    tm[860:870] = np.inf
+    d[870:900] *= rng.choice([1e-8, 1e6, 1e-20], (30, 1))
+    for k, v in ((900, np.nan), (910, np.inf), (920, -np.inf)):
+        o[k:k + 3, 0] = v
+        o[k + 3:k + 6, 2] = v
+        d[k + 6:k + 8, 1] = v
+        t0[k + 8] = v
+        tm[k + 9] = v
+    return abi.HostRays.from_arrays(o.astype(f32), d.astype(f32), t0.astype(f32), tm.astype(f32))
+
+
+@pytest.mark.parametrize("kind", ["tris1", "tris2", "tris3", "tris5", "tris17", "tris4000", "stacked", "blob_spheres",
+                                  "pathlines"])
+def test_the_wide_walk_gives_the_binary_walks_hits(hip, kind):
+    from galaxy_amd import lib as glib
+    L = glib.lib()
+    B = scenes.build_scene(hip, _scene(kind))
+    hr = _rays()
+    for k, typ in ((1, abi.RAY_SHADOW), (2, abi.RAY_AO)):
+        hr["type"][k::5] = typ
+    geom, prim = glib.DeviceArray(4 * hr.n), glib.DeviceArray(4 * hr.n)
+    glib.check(L.gxy_model_set_hit_output(B.vis.model, geom.ptr, prim.ptr))
+    got = []
+    try:
+        for width, stack, waves in ((2, 16, 0), (2, 0, 8), (4, 0, 0), (2, 0, 0)):
+            glib.check(L.gxy_set_bvh_width(width))
+            glib.check(L.gxy_set_geometry_stack(stack))
+            glib.check(L.gxy_set_geometry_waves(waves))
+            d = glib.DeviceRays.from_host(hr)
+            assert hip.trace(B.vis, d) == ""
+            g = d.download()
+            got.append([g[f].view(np.int32) for f in abi.FIELDS] + [geom.to_host(np.int32, hr.n),
+                                                                   prim.to_host(np.int32, hr.n)])
+    finally:
+        L.gxy_set_bvh_width(2)
+        L.gxy_set_geometry_stack(0)
+        L.gxy_set_geometry_waves(0)
+        L.gxy_model_set_hit_output(B.vis.model, None, None)
+    assert (got[0][-2] >= 0).any()
+    for other in got[1:]:
+        for f, a, b in zip(abi.FIELDS + ("geom", "prim"), got[0], other):
+            bad = np.nonzero(a != b)[0]
+            assert len(bad) == 0, (kind, f, bad[:5])
+
+
+def test_mixed_scenes_take_the_same_walks(hip):
+    """A volume with a mesh inside (the kernel that both marches and walks)."""
+    from galaxy_amd import lib as glib
+    L = glib.lib()
+    sc = workloads.unit_volume_scene(24, 4)
+    sc.meshes = [scenes.blob_mesh(4000, 9)]
+    B = scenes.build_scene(hip, sc)
+    hr = _rays()
+    got = []
+    try:
+        for width, stack in ((2, 16), (4, 0)):
+            glib.check(L.gxy_set_bvh_width(width))
+            glib.check(L.gxy_set_geometry_stack(stack))
+            d = glib.DeviceRays.from_host(hr.subset(np.arange(900)))
+            assert hip.trace(B.vis, d) == ""
+            g = d.download()
+            got.append([g[f].view(np.int32) for f in abi.FIELDS])
+    finally:
+        L.gxy_set_bvh_width(2)
+        L.gxy_set_geometry_stack(0)
+    assert all(np.array_equal(a, b) for a, b in zip(*got))
