@@ -146,6 +146,13 @@ struct DGeomShade {
   DTF tf;
 };
 
+// The sample counter is spread over this many 64-bit counters, 128 bytes apart:
+// additions to one address complete one after another (about 15 ns each), so
+// the waves of a large launch would queue on a single counter.
+#define GXY_COUNT_SLOTS 64
+#define GXY_COUNT_STRIDE 16
+#define GXY_COUNT_BYTES (GXY_COUNT_SLOTS * GXY_COUNT_STRIDE * 8)
+
 struct TraceParams {
   int nvv;
   int integrate;
@@ -157,7 +164,7 @@ struct TraceParams {
   float opaque_alpha;  // early termination: alpha above this is opaque (0.999)
   DVolVis vv[GXY_MAX_VOLVIS];
   DModel model;
-  unsigned long long *sample_count;    // volume samples are added here, one atomic per wave (may be null)
+  unsigned long long *sample_count;    // volume samples are added here: GXY_COUNT_SLOTS counters (may be null)
   int *hit_geom;                       // side-band geomID per ray, may be null
   int *hit_prim;
   // a launch queued before its list's size is known: when dn is set, the

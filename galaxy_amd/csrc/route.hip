@@ -301,13 +301,17 @@ __global__ __launch_bounds__(GXY_BLOCK) void k_sampler_write(RayList_ispc R, int
 __global__ void k_add_count(int *count, const int *add) { *count += *add; }
 
 // The values the host waits for after a list, written straight into mapped
-// host memory: out[0..na) = a, out[16] = *b, out[18..19] = *c (64-bit), and
-// out[32] = seq once the others are visible to the host.
+// host memory: out[0..na) = a, out[16] = *b, out[18..19] = the sum of the
+// GXY_COUNT_SLOTS counters at c (64-bit), and out[32] = seq once the others are
+// visible to the host.
 __global__ void k_readback(const int *a, int na, const int *b, const unsigned long long *c, int *out, int seq) {
   const int t = threadIdx.x;
   if (t < na) out[t] = a[t];
   if (t == 16 && b) out[16] = *b;
-  if (t == 18 && c) *(unsigned long long *)(out + 18) = *c;
+  if (c) {
+    const unsigned long long v = wave_sum_u64(t < GXY_COUNT_SLOTS ? c[t * GXY_COUNT_STRIDE] : 0);
+    if (t == 0) *(unsigned long long *)(out + 18) = v;
+  }
   __threadfence_system();
   __syncthreads();
   if (t == 0) {

@@ -63,7 +63,7 @@ struct PendingEv {
 };
 
 // An execution context: one HIP stream (default priority), its device
-// counters ([0] samples), and a cache of freed device blocks that are reused
+// counters (volume samples, GXY_COUNT_SLOTS of them), and a cache of freed device blocks that are reused
 // only on this stream (stream order makes the reuse safe without a sync).
 struct Ctx {
   hipStream_t stream = nullptr;
@@ -365,9 +365,9 @@ static int ensure_init() {
   G.uv = (float *)dalloc(sizeof UV);
   if (!G.uv) return -1;
   HIPCHK(hipMemcpy(G.uv, UV, sizeof UV, hipMemcpyHostToDevice));
-  G.def.counters = (unsigned long long *)dalloc(8 * sizeof(unsigned long long));
+  G.def.counters = (unsigned long long *)dalloc(GXY_COUNT_BYTES);
   if (!G.def.counters) return -1;
-  HIPCHK(hipMemsetAsync(G.def.counters, 0, 8 * sizeof(unsigned long long), S()));
+  HIPCHK(hipMemsetAsync(G.def.counters, 0, GXY_COUNT_BYTES, S()));
   return 0;
 }
 #define INIT_OR(ret) \
@@ -651,7 +651,7 @@ GXY_EXPORT void *gxy_context_create(void) {
   }
   Ctx *prev = t_ctx;
   t_ctx = c;
-  c->counters = (unsigned long long *)dalloc(8 * sizeof(unsigned long long));
+  c->counters = (unsigned long long *)dalloc(GXY_COUNT_BYTES);
   // the readback area now, so that no later call on this context allocates it
   if (!c->counters || !readback_area(*c)) {
     dfree_stream_ordered(c->counters);
@@ -666,7 +666,7 @@ GXY_EXPORT void *gxy_context_create(void) {
     return nullptr;
   }
   t_ctx = prev;
-  hipMemsetAsync(c->counters, 0, 8 * sizeof(unsigned long long), c->stream);
+  hipMemsetAsync(c->counters, 0, GXY_COUNT_BYTES, c->stream);
   hipStreamSynchronize(c->stream);
   std::lock_guard<std::recursive_mutex> lk(G.mu);
   G.contexts.insert(c);
@@ -1755,7 +1755,7 @@ GXY_EXPORT int gxy_model_set_hit_output(void *model, int *g, int *p) {
 }
 
 // Trace (or sampler) launch; its volume samples are added to the context's
-// sample counter (counters[0]) by the kernel's waves.
+// sample counters by the kernel's waves.
 static int trace_launch(TraceParams P, const RayList_ispc &R, int n, bool sampler) {
   if (n <= 0) return 0;
   const bool pl = !sampler && G.trace_kind == 1 && P.nvv >= 1 && !P.has_model;
@@ -2523,7 +2523,7 @@ static int process_list(LoopCtx &C, RayListObj *L, int prio, bool owned) {
 }
 
 static int run_loop(LoopCtx &C, int n, const RayList_ispc &rays, RayListObj *adopt = nullptr) {
-  if (!C.have_base) HIPCHK(hipMemsetAsync(CX().counters, 0, 8 * sizeof(unsigned long long), S()));
+  if (!C.have_base) HIPCHK(hipMemsetAsync(CX().counters, 0, GXY_COUNT_BYTES, S()));
   if (adopt && n <= C.maxlist) {
     // the caller's list is processed in place (it is the loop's to consume)
     C.q.push_back({adopt, 3});

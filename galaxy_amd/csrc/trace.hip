@@ -293,15 +293,6 @@ hipError_t launch_trace_pl(const TraceParams &P, const RayList_ispc &R, int n, i
   return hipErrorInvalidValue;
 }
 
-// ------------------------------------------------------------- sampler kernel
-template <int NV, int SM>
-__global__ __launch_bounds__(GXY_BLOCK) void k_sampler(TraceParams P, RayList_ispc R, int n) {
-  const int i = blockIdx.x * GXY_BLOCK + threadIdx.x;
-  unsigned long long nsamp = 0;
-  if (i < n) nsamp = sample_one<NV, SM>(P, R, i);
-  if (P.sample_count) wave_add_count(nsamp, P.sample_count);
-}
-
 // ------------------------------------------------------------- launchers
 // one volume with a bricked copy: the variant for its addressing (32-bit
 // offsets when the copy spans under 4 GiB) and the occupancy request
@@ -375,34 +366,6 @@ hipError_t launch_trace(const TraceParams &P, const RayList_ispc &R, int n, int 
     case 4: return launch_trace_nv<4>(P, R, n, wpe, stack, s, gwaves, bs);
   }
   return hipErrorInvalidValue;
-}
-
-hipError_t launch_sampler(const TraceParams &P, const RayList_ispc &R, int n, hipStream_t s) {
-  if (n <= 0) return hipSuccess;
-  dim3 g((n + GXY_BLOCK - 1) / GXY_BLOCK), b(GXY_BLOCK);
-  bool small = P.nvv > 0;
-  for (int v = 0; v < P.nvv && v < GXY_MAX_VOLVIS; v++) small = small && P.vv[v].vol.small;
-  if (P.nvv == 1 && P.vv[0].vol.brick) {
-    switch (sm_of(P.vv[0].vol)) {
-      case 4: hipLaunchKernelGGL((k_sampler<1, 4>), g, b, 0, s, P, R, n); break;
-      case 8: hipLaunchKernelGGL((k_sampler<1, 8>), g, b, 0, s, P, R, n); break;
-      case 12: hipLaunchKernelGGL((k_sampler<1, 12>), g, b, 0, s, P, R, n); break;
-      default: hipLaunchKernelGGL((k_sampler<1, 16>), g, b, 0, s, P, R, n); break;
-    }
-    return hipGetLastError();
-  }
-  switch (P.nvv * 2 + (small ? 1 : 0)) {
-    case 2: hipLaunchKernelGGL((k_sampler<1, -1>), g, b, 0, s, P, R, n); break;
-    case 3: hipLaunchKernelGGL((k_sampler<1, 1>), g, b, 0, s, P, R, n); break;
-    case 4: hipLaunchKernelGGL((k_sampler<2, -1>), g, b, 0, s, P, R, n); break;
-    case 5: hipLaunchKernelGGL((k_sampler<2, 1>), g, b, 0, s, P, R, n); break;
-    case 6: hipLaunchKernelGGL((k_sampler<3, -1>), g, b, 0, s, P, R, n); break;
-    case 7: hipLaunchKernelGGL((k_sampler<3, 1>), g, b, 0, s, P, R, n); break;
-    case 8: hipLaunchKernelGGL((k_sampler<4, -1>), g, b, 0, s, P, R, n); break;
-    case 9: hipLaunchKernelGGL((k_sampler<4, 1>), g, b, 0, s, P, R, n); break;
-    default: return hipErrorInvalidValue;
-  }
-  return hipGetLastError();
 }
 
 }  // namespace gxy
