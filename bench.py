@@ -572,7 +572,7 @@ def main():
     if w > 6 and not one:
         w = 6                               # 17 / 18 act as 16 beyond one bricked volume and isovalue
     bs = kcfg[1].value if (one and w == 6 and kcfg[1].value in (64, 128)) else 256
-    roof["kernel"] = ("k_trace_pl<1>" if k == 1 else
+    roof["kernel"] = ("k_trace_pl<1>" if k == 1 else "k_march" if k == 0 else
                       "k_trace<1,false,%d,%d,%d,%d>" % (w, sm, 1 if one else 8, bs))
     roof["volume_layout"] = lay
     roof["kernel_ms_per_launch"] = round(tr_ms / max(1, tr_n), 4)

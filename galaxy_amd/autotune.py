@@ -5,8 +5,8 @@ not change; only how rays are mapped onto lanes does), so the tuner only
 measures: it renders the caller's frame once per candidate with HIP-event
 timing of the trace kernel enabled and keeps the fastest.
 
-Candidates: one ray per work-item (kind 0, and its 5- and 6-waves-per-SIMD
-occupancy variants 15 and 16), or persistent lanes (kind 1) with a per-wave
+Candidates: the library's choice of lanes per ray (kind 0), one ray per
+work-item at 5 or 6 waves per SIMD (kinds 15 and 16), or persistent lanes (kind 1) with a per-wave
 chunk of 128 or 256 consecutive rays and a refill threshold of 16 or 32 idle
 lanes out of 64.  (Measured on the volume-render frame: the persistent form
 was 2-5x slower than one ray per work-item; it stays a candidate for other

@@ -63,6 +63,7 @@ struct DTF {
   float sc, so;   // (nc-1)/(hi-lo), (no-1)/(hi-lo)
   float xc, xo;   // nc-1, no-1 as floats (the clamp bounds of the table coordinate)
   float lo2, hsc, hso;  // 2 lo, sc / 2, so / 2: coordinates of a doubled value
+  int bounded;          // every table entry is under 1e30 in magnitude (no infinity, no NaN)
 };
 
 struct DVolVis {

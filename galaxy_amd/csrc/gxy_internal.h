@@ -51,6 +51,10 @@ struct CameraParams {
 hipError_t launch_trace(const TraceParams &P, const RayList_ispc &R, int n, int wpe, int stack, hipStream_t s,
                         int gwaves = 0, int bs = GXY_BLOCK);
 int trace_block_size(const TraceParams &P, int wpe, int bs);
+// one volume, several lanes per ray (launch_trace calls it): false when the list
+// is for the one-lane march
+bool launch_march(const TraceParams &P, const RayList_ispc &R, int n, hipStream_t s);
+int march_lanes(int n, int dn_mul, float steps);
 // the same for geometry without volumes (launch_trace calls it)
 hipError_t launch_trace_geom(const TraceParams &P, const RayList_ispc &R, int n, int stack, int gwaves,
                              hipStream_t s);

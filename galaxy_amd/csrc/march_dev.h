@@ -130,4 +130,251 @@ __device__ __forceinline__ unsigned sample_group(const TraceParams &P, const Ray
   return nsamp;
 }
 
+// the value of lane k of the group, in all its lanes
+template <int G>
+__device__ __forceinline__ float dpp_bcast(float v, int k) {
+  const int i = __float_as_int(v);
+  int r = i;
+  // (k is a constant once the loops around the calls are unrolled)
+#define GXY_BC(K)                                                                            \
+  if (k == K) {                                                                              \
+    if (G == 2) r = __builtin_amdgcn_mov_dpp(i, (K & 1) ? 0xF5 : 0xA0, 0xf, 0xf, false);     \
+    else if (G == 4) r = __builtin_amdgcn_mov_dpp(i, (K & 3) * 0x55, 0xf, 0xf, false);       \
+    else if (G == 16) r = __builtin_amdgcn_mov_dpp(i, 0x150 + (K & 15), 0xf, 0xf, false);    \
+    else {                                                                                   \
+      r = __builtin_amdgcn_update_dpp(i, i, 0x150 + (K & 7), 0xf, 0x3, false);               \
+      r = __builtin_amdgcn_update_dpp(r, i, 0x158 + (K & 7), 0xf, 0xc, false);               \
+    }                                                                                        \
+  }
+  GXY_BC(0) GXY_BC(1) GXY_BC(2) GXY_BC(3) GXY_BC(4) GXY_BC(5) GXY_BC(6) GXY_BC(7)
+  GXY_BC(8) GXY_BC(9) GXY_BC(10) GXY_BC(11) GXY_BC(12) GXY_BC(13) GXY_BC(14) GXY_BC(15)
+#undef GXY_BC
+  return __int_as_float(r);
+}
+
+// trace_one of one volume without geometry, with G lanes per ray (every lane of
+// the group calls it for the same ray, the k-th after ray `first`, which is
+// uniform over the wave).  Position T_0 is the entry point, T_1 = T_0 + epsilon,
+// T_k+1 = min(T_k + step, tTermination); the samples at T_k are taken side by
+// side, and their colours are composited in order: each round every lane applies
+// the samples of its group's lanes up to its own, one after another, to the
+// colour at the round's start, so that lane j holds the colour after its sample.
+// The first lane whose sample crosses an isovalue or makes the ray opaque ends
+// the march and writes the ray.  (A lane past it, or one whose sample has no
+// opacity, applies weight 0, which changes nothing as long as the tables and
+// the ray's alpha are finite: the launcher checks the tables, `odd` the rays.)
+// shade: the rays are primary (a wave with both kinds runs this once for each).
+template <int G, int SM, int MI, bool shade>
+__device__ __forceinline__ unsigned trace_group(const TraceParams &P, const RayList_ispc &R, const int first,
+                                                const unsigned i, const float *s_col, const float *s_op) {
+  const int j = group_lane<G>();
+  const DVolVis &VV = P.vv[0];
+  const DVolume &V = VV.vol;
+  const DTF &T = VV.tf;
+  unsigned nsamp = 0;
+  float ray_t0 = gptr(R.t + first)[i];
+  float ray_t = gptr(R.tMax + first)[i];
+  float cr = gptr(R.r + first)[i], cg = gptr(R.g + first)[i], cb = gptr(R.b + first)[i], ca = gptr(R.o + first)[i];
+  // Only what the march needs stays in registers through it (six waves per
+  // SIMD): the ray's origin and direction, its slice's normal and colour are
+  // read or formed again afterwards.
+  VoxRay VR;
+  float tEntry, tExitVolume;
+  int slice = -1;
+  {
+    const f3 org = ray_org(R, first, i), dir = ray_dir(R, first, i);
+    box_clip(org, dir, P.blo, P.bhi, tEntry, tExitVolume);
+    if (tEntry < ray_t0) tEntry = ray_t0;
+    else if (tEntry > ray_t0) ray_t0 = tEntry;
+    ray_t = mnf(ray_t, tExitVolume);
+    // LookForSliceHit (TraceRays.ispc:143-250)
+    for (int m = 0; m < VV.nSlices; m++) {
+      const f3 pn = mk3(VV.slices[4 * m], VV.slices[4 * m + 1], VV.slices[4 * m + 2]);
+      const float denom = dot3(dir, pn);
+      if (fabsf(denom) > 0.0001f) {
+        const float t = (VV.slices[4 * m + 3] - dot3(org, pn)) / denom;
+        if (t >= ray_t0 && t <= ray_t) {
+          ray_t = t;
+          slice = m;
+        }
+      }
+    }
+    VR = vox_ray(V, org, dir);
+  }
+
+  float tTermination = ray_t;
+  bool owner = j == G - 1, hit_iso = false;
+  float hit_sample = 0.f;
+  if (P.integrate && tEntry <= tTermination && !opaque_of(cr, cg, cb, ca, P.opaque_alpha)) {
+    const float step = P.step, eps = P.eps;
+    const bool odd = __builtin_amdgcn_ballot_w64(!(fabsf(ca) < 1e30f)) != 0;
+    const float T1 = tEntry + eps;
+    const float lim = (T1 > tEntry && T1 <= tTermination) ? tTermination : tEntry;
+    float t = j == 0 ? tEntry : T1, tp = tEntry;
+#pragma unroll
+    for (int k = 2; k < G; k++)
+      if (k <= j) {
+        tp = t;
+        t += step;
+      }
+    t = __builtin_fminf(t, lim);
+    tp = __builtin_fminf(tp, lim);
+    VFetch F = vox_fetch<SM>(V, VR, t);
+    float sEnd = 0.f, tThis;
+    float fstep = j == 0 ? eps : step;   // (the step after T_0 is epsilon)
+    nsamp = j == 0 ? 1u : 0u;
+    int iter = 0, hI, end;
+    bool go;
+    do {
+      if (VV.dvr) {
+        // the colour after the last round
+        cr = dpp_bcast<G>(cr, G - 1);
+        cg = dpp_bcast<G>(cg, G - 1);
+        cb = dpp_bcast<G>(cb, G - 1);
+        ca = dpp_bcast<G>(ca, G - 1);
+      }
+      // this round's samples; the next round's gathers before they are used
+      float tn, tpn;
+      group_advance<G>(t, fstep, step, lim, tn, tpn);
+      fstep = step;
+      float s = vol_finish_fma(F);
+      F = vox_fetch<SM>(V, VR, tn);
+      const float sl0 = dpp_prev(s);
+      const float sl = j == 0 ? sEnd : sl0;
+      sEnd = dpp_last_to_first<G>(s);
+      const bool step_ok = t > tp;
+      const bool live = step_ok && tp >= eps;
+      // LookForIsoHit: the last matching isovalue in list order wins
+      bool ih = false;
+#pragma unroll
+      for (int m = 0; m < MI; m++)
+        if (m < VV.nIso) {
+          const float iso = VV.iso[m];
+          if (((iso >= sl) && (iso < s)) || ((iso <= sl) && (iso > s))) {
+            ih = live;
+            hit_sample = iso;
+          }
+        }
+      tThis = t;
+      hI = G;
+      const unsigned long long im = __builtin_amdgcn_ballot_w64(ih);
+      if (im) {
+        const unsigned b = group_bits<G>(im);
+        hI = b ? __builtin_ctz(b) : G;
+        if (j == hI) {
+          tThis = tp + ((hit_sample - sl) / (s - sl)) * (t - tp);
+          s = vox_sample<SM>(V, VR, tThis);
+        }
+      }
+      end = hI;
+      if (VV.dvr) {
+        const float d = (sl + s) - T.lo2;
+        float w = tf_opacity_d2(s_op, T, d);
+        w = live && j <= hI && w > 0.f ? clamp01f(w * V.irate) : 0.f;
+        const bool some = w != 0.f;
+        if (__builtin_amdgcn_ballot_w64(some)) {
+          if (shade) {
+            const f3 sc = tf_color_num_d2(s_col, T, d);
+            if (!odd) {
+#pragma unroll
+              for (int k = 0; k < G; k++) {
+                const float wk0 = dpp_bcast<G>(w, k);
+                const float wk = k <= j ? wk0 : 0.f;
+                const float a = 1.0f - ca, aw = a * wk;
+                cr = __builtin_fmaf(aw, dpp_bcast<G>(sc.x, k), cr);
+                cg = __builtin_fmaf(aw, dpp_bcast<G>(sc.y, k), cg);
+                cb = __builtin_fmaf(aw, dpp_bcast<G>(sc.z, k), cb);
+                ca = __builtin_fmaf(a, wk, ca);
+              }
+            } else {
+#pragma unroll
+              for (int k = 0; k < G; k++) {
+                const float wk = dpp_bcast<G>(w, k);
+                const f3 sk = mk3(dpp_bcast<G>(sc.x, k), dpp_bcast<G>(sc.y, k), dpp_bcast<G>(sc.z, k));
+                if (k <= j && wk != 0.f) composite(cr, cg, cb, ca, sk, wk);
+              }
+            }
+          } else {
+            const float f = some ? 1.0f - ((tThis - tp) * P.istep) * w : 1.0f;
+#pragma unroll
+            for (int k = 0; k < G; k++) {
+              const float fk0 = dpp_bcast<G>(f, k);
+              const float fk = k <= j ? fk0 : 1.f;
+              cr *= fk; cg *= fk; cb *= fk; ca *= fk;
+            }
+          }
+          const unsigned long long om =
+              __builtin_amdgcn_ballot_w64(step_ok && opaque_of(cr, cg, cb, ca, P.opaque_alpha));
+          if (om) {
+            const unsigned b = group_bits<G>(om);
+            end = b ? min(hI, (int)__builtin_ctz(b)) : hI;
+          }
+        }
+      }
+      nsamp += (step_ok && j <= end) ? 1u : 0u;
+      // on, unless an event ended the march or the position after this round's
+      // last (lane 0's next) no longer advances
+      iter += G;
+      const float tl = dpp_bcast<G>(t, G - 1);
+      go = end == G && __builtin_fminf(tl + step, lim) > tl && iter < GXY_MAX_MARCH;
+      t = tn;
+      tp = tpn;
+    } while (go);
+    if (end < G) {
+      // lane `end` ended the march: by an isovalue when it is hI
+      owner = j == end;
+      hit_iso = end == hI;
+      tTermination = tThis;
+      nsamp += owner && hit_iso ? 1u : 0u;
+    }
+  }
+  asm volatile("" ::: "memory");   // the fields are read again, not kept
+  f3 nrm = mk3(0.f, 0.f, 0.f), col = nrm;
+  bool surface_opaque = slice >= 0;
+  if (slice >= 0) {
+    const f3 org = ray_org(R, first, i), dir = ray_dir(R, first, i);
+    const f3 pn = mk3(VV.slices[4 * slice], VV.slices[4 * slice + 1], VV.slices[4 * slice + 2]);
+    nrm = dot3(dir, pn) > 0 ? neg3(pn) : pn;
+    if (shade && !hit_iso) col = tf_color(s_col, T, vol_sample_t<SM>(V, add3(org, scl3(ray_t, dir))));
+  }
+  if (shade && hit_iso) {
+    // LookForIsoHit shading (TraceRays.ispc:284-307): the four samples of the
+    // forward-difference gradient side by side in the group's lanes
+    surface_opaque = true;
+    const f3 org = ray_org(R, first, i), dir = ray_dir(R, first, i);
+    const unsigned ob = group_bits<G>(__builtin_amdgcn_ballot_w64(owner));
+    const float ht = __shfl(tTermination, ((threadIdx.x & 63) & ~(G - 1)) + __builtin_ctz(ob), 64);
+    const f3 p = add3(org, scl3(ht, dir));
+    float g[4];
+#pragma unroll
+    for (int q = 0; q < 4; q += G) {
+      const int a = q + j;
+      const float v = vol_sample_t<SM>(
+          V, add3(p, mk3(a == 1 ? V.sp[0] : 0.f, a == 2 ? V.sp[1] : 0.f, a == 3 ? V.sp[2] : 0.f)));
+#pragma unroll
+      for (int k = 0; k < G && q + k < 4; k++) g[q + k] = dpp_bcast<G>(v, k);
+    }
+    nrm = safe_normalize3(mk3((g[1] - g[0]) / V.sp[0], (g[2] - g[0]) / V.sp[1], (g[3] - g[0]) / V.sp[2]));
+    if (dot3(dir, nrm) > 0) nrm = neg3(nrm);
+    col = tf_color(s_col, T, hit_sample);
+  }
+  if (!owner) return nsamp;
+  gptr(R.r + first)[i] = cr; gptr(R.g + first)[i] = cg; gptr(R.b + first)[i] = cb; gptr(R.o + first)[i] = ca;
+  int term = opaque_of(cr, cg, cb, ca, P.opaque_alpha) ? RAY_OPAQUE : 0;
+  if (slice >= 0 || hit_iso) {
+    term |= RAY_SURFACE;
+    if (surface_opaque) term |= RAY_OPAQUE;
+    gptr(R.sr + first)[i] = col.x; gptr(R.sg + first)[i] = col.y; gptr(R.sb + first)[i] = col.z;
+    gptr(R.so + first)[i] = 1.0f;
+    gptr(R.nx + first)[i] = nrm.x; gptr(R.ny + first)[i] = nrm.y; gptr(R.nz + first)[i] = nrm.z;
+  } else if (tTermination == tExitVolume) {
+    term |= RAY_BOUNDARY;
+  } else if (tTermination == gptr(R.tMax + first)[i]) {
+    term |= RAY_TIMEOUT;
+  }
+  gptr(R.t + first)[i] = tTermination;
+  gptr(R.term + first)[i] = term;
+  return nsamp;
+}
+
 }  // namespace gxy

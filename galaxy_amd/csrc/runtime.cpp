@@ -1110,6 +1110,10 @@ static void *tf_make(std::vector<float> col, std::vector<float> op, float lo, fl
   t->d.lo2 = 2.f * lo;
   t->d.hsc = 0.5f * t->d.sc;
   t->d.hso = 0.5f * t->d.so;
+  t->d.bounded = 1;
+  for (const std::vector<float> *tab : {&dcol, &dop})
+    for (float v : *tab)
+      if (!(std::fabs(v) < 1e30f)) t->d.bounded = 0;
   std::lock_guard<std::recursive_mutex> lk(G.mu);
   G.tfs.insert(t);
   return t;

@@ -358,6 +358,8 @@ static hipError_t launch_trace_nv(const TraceParams &P, const RayList_ispc &R, i
 hipError_t launch_trace(const TraceParams &P, const RayList_ispc &R, int n, int wpe, int stack, hipStream_t s,
                         int gwaves, int bs) {
   if (n <= 0) return hipSuccess;
+  // (an occupancy asked for by the caller names a one-ray-per-item kernel)
+  if (wpe == 0 && launch_march(P, R, n, s)) return hipGetLastError();
   switch (P.nvv) {
     case 0: return launch_trace_nv<0>(P, R, n, wpe, stack, s, gwaves, bs);
     case 1: return launch_trace_nv<1>(P, R, n, wpe, stack, s, gwaves, bs);

@@ -191,14 +191,15 @@ size_t      gxy_device_bytes_in_use(void);
 int         gxy_set_opacity_threshold(float alpha);
 float       gxy_get_opacity_threshold(void);
 /* Launch configuration of the volume-only trace (no reference counterpart):
- * kind 0 = one ray per work-item; 15 / 16 / 17 / 18 = the same kernel compiled
- * for at least 5 / 6 / 7 / 8 waves per SIMD (17 and 18 for one bricked volume
- * with at most one isovalue, 16 otherwise), where `chunk` 64 or 128 selects that
- * many work-items per workgroup for kind 16 on one bricked volume with at most
- * one isovalue (256 otherwise); kind 1 = persistent lanes, each wave owning
- * `chunk` consecutive rays (multiple of 64) and refilling idle lanes once
- * `refill` (1..64) of them are idle.  Results are identical for every setting;
- * galaxy_amd/autotune.py picks the fastest. */
+ * kind 0 (default) = for one volume, 2, 4 or 16 lanes per ray by the list's size
+ * against the length of its rays, one ray per work-item elsewhere; 15 / 16 / 17 /
+ * 18 = one ray per work-item compiled for at least 5 / 6 / 7 / 8 waves per SIMD
+ * (17 and 18 for one bricked volume with at most one isovalue, 16 otherwise),
+ * where `chunk` 64 or 128 selects that many work-items per workgroup for kind 16
+ * on one bricked volume with at most one isovalue (256 otherwise); kind 1 =
+ * persistent lanes, each wave owning `chunk` consecutive rays (multiple of 64)
+ * and refilling idle lanes once `refill` (1..64) of them are idle.  Results are
+ * identical for every setting; galaxy_amd/autotune.py picks the fastest. */
 int         gxy_set_trace_config(int kind, int chunk, int refill);
 /* Binary BVH walk of geometry-only traces (no reference counterpart) with 16 /
  * 24 / 32 traversal stack entries in LDS (deeper entries in private memory);

@@ -68,3 +68,73 @@ def test_sampler_lanes_take_the_one_ray_march(hip, n, edge, layout, rate):
         assert np.array_equal(g[f].view(np.int32), r[f].view(np.int32)), f
     if n > 1000 and edge > 3 and rate < 1:
         assert 0.05 < np.mean(g["term"] == abi.RAY_SURFACE) < 0.95
+
+
+def _trace(hip, B, hr, kind):
+    from galaxy_amd import lib as glib
+    L = glib.lib()
+    saved = [C.c_int() for _ in range(3)]
+    L.gxy_get_trace_config(*[C.byref(x) for x in saved])
+    glib.check(L.gxy_set_trace_config(kind, 256, 32))
+    try:
+        d = glib.DeviceRays.from_host(hr)
+        assert hip.trace(B.vis, d) == ""
+        return d.download()
+    finally:
+        L.gxy_set_trace_config(*[x.value for x in saved])
+
+
+def _mixed_rays(n, seed):
+    """Primary, shadow and AO rays with colours in hand, some of them odd."""
+    hr = _rays(n, seed)
+    rng = np.random.default_rng(seed)
+    hr["type"] = rng.choice([abi.RAY_PRIMARY, abi.RAY_SHADOW, abi.RAY_AO], n)
+    if n > 200:
+        hr["type"][:128] = abi.RAY_PRIMARY
+    for f in "rgb":
+        hr[f] = rng.uniform(-0.3, 0.3, n)
+    hr["o"] = rng.uniform(0, 0.5, n)
+    for f, k in (("o", 5), ("r", 6), ("o", 7), ("g", 8)):
+        for v, q in ((np.inf, 0), (-np.inf, 100), (np.nan, 200)):
+            hr[f][k + q::1000] = v
+    for f in ("sr", "sg", "sb", "so", "nx", "ny", "nz"):
+        hr[f] = 0.25
+    return hr
+
+
+# 16 lanes up to 2^16 rays; at 16 march steps across the box 4096 rays per step
+# (two lanes) and 5.6 K (one), at 64 steps 1 K (four)
+@pytest.mark.parametrize("n,edge", [(1, 3), (15, 9), (257, 33), (65536, 9), (65537, 9), (90001, 9), (65537, 33)])
+@pytest.mark.parametrize("layout,isos,slices,dvr", [(0, 1, 0, True), (4, 1, 0, True), (8, 0, 1, True), (0, 2, 2, True),
+                                                    (4, 2, 0, False), (8, 1, 1, True), (0, 0, 1, False)])
+def test_lanes_per_ray_give_the_one_lane_march(hip, n, edge, layout, isos, slices, dvr):
+    from galaxy_amd import lib as glib
+    sc = _volume(edge, 6)
+    vv = sc.volume_vis[0]
+    vv.isovalues, vv.volume_render = vv.isovalues[:isos], dvr
+    vv.slices = np.array([[0, 0, 1, 0.4], [0.6, 0.8, 0, 0.7]], f32)[:slices]
+    B = scenes.build_scene(hip, sc)
+    if layout:
+        glib.check(glib.lib().gxy_volume_set_layout(B.handles[0], layout))
+    hr = _mixed_rays(n, 11 + n)
+    a, b = _trace(hip, B, hr, 0), _trace(hip, B, hr, 16)
+    for f in abi.FIELDS:
+        x, y = a[f].view(np.int32), b[f].view(np.int32)
+        if a[f].dtype == f32:      # (the bits of a NaN are not part of the result)
+            x, y = np.where(np.isnan(a[f]), 0, x), np.where(np.isnan(b[f]), 0, y)
+            assert np.array_equal(np.isnan(a[f]), np.isnan(b[f])), f
+        assert np.array_equal(x, y), (f, np.nonzero(x != y)[0][:5])
+
+
+def test_unbounded_tables_keep_the_one_lane_march(hip):
+    """A table with an infinity or a NaN: weights of zero would spread it."""
+    from galaxy_amd import lib as glib
+    sc = _volume(17, 6)
+    for bad in (np.inf, np.nan):
+        vv = sc.volume_vis[0]
+        vv.colormap = np.array([[0, 0.2, 0.3, 0.4], [0.8, 0.5, 0.6, 0.7], [1.0, bad, 0.1, 0.1]], f32)
+        B = scenes.build_scene(hip, sc)
+        hr = _mixed_rays(4000, 21)
+        a, b = _trace(hip, B, hr, 0), _trace(hip, B, hr, 16)
+        for f in abi.FIELDS:
+            assert np.array_equal(a[f], b[f], equal_nan=a[f].dtype == f32), f
