@@ -1,4 +1,5 @@
-// march_dev.h — volume marches with several lanes per ray.
+// march_dev.h — volume marches with several lanes per ray, shared by the
+// one-list kernels (sampler.hip, march.hip) and the batched kernels (batch.hip).
 //
 // One lane per ray leaves a march with a serial chain per sample (gathers, the
 // interpolation, the test) and 64 rays' samples spread over 64 places of the
@@ -14,6 +15,13 @@
 #include "trace_dev.h"
 
 namespace gxy {
+
+// LDS writes of one wave become visible to its other lanes
+__device__ __forceinline__ void wave_lds_sync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
 
 // Lane j of its group of G (G = 2, 4, 8 or 16 adjacent lanes).
 template <int G>
@@ -51,85 +59,6 @@ __device__ __forceinline__ void group_advance(float t, float first_step, float s
   tpn = __builtin_fminf(tpn, lim);
 }
 
-// sample_one of one volume with G lanes per ray (every lane of the group calls
-// it with the same i).  Position T_0 is the entry point and T_k+1 = min(T_k +
-// step, tExit); the march ends where that no longer advances.
-template <int G, int SM>
-__device__ __forceinline__ unsigned sample_group(const TraceParams &P, const RayList_ispc &R, const int i) {
-  const int j = group_lane<G>();
-  const DVolume &V = P.vv[0].vol;
-  f3 org = mk3(gptr(R.ox)[i], gptr(R.oy)[i], gptr(R.oz)[i]);
-  f3 dir = mk3(gptr(R.dx)[i], gptr(R.dy)[i], gptr(R.dz)[i]);
-  const float rt = gptr(R.t)[i];
-  if (dir.x == 0.f) dir.x = 1e-6f;
-  if (dir.y == 0.f) dir.y = 1e-6f;
-  if (dir.z == 0.f) dir.z = 1e-6f;
-  float tEntry, tExit;
-  box_clip(org, dir, P.blo, P.bhi, tEntry, tExit);
-  if (tEntry < rt) tEntry = rt;
-  const float step = P.step, iso = P.vv[0].iso[0];
-  const VoxRay VR = vox_ray(V, org, dir);
-  // the first step is not cut at the exit: a ray whose first step leaves takes
-  // no step at all (its chain stays at the entry)
-  const bool go0 = tEntry + step <= tExit;
-  const float lim = go0 ? tExit : tEntry;
-  float t = tEntry, tp = tEntry;
-#pragma unroll
-  for (int k = 1; k < G; k++)
-    if (k <= j) {
-      tp = t;
-      t += step;
-    }
-  t = __builtin_fminf(t, lim);
-  tp = __builtin_fminf(tp, lim);
-  VFetch F = vox_fetch<SM>(V, VR, t);
-  float sEnd = 0.f;   // lane 0: the last lane's sample of the round before
-  unsigned nsamp = j == 0 ? 1u : 0u;
-  // (round `iter` holds positions iter .. iter + G - 1; at most GXY_MAX_MARCH
-  // samples after the first, a multiple of G)
-  for (int iter = 0;; iter += G) {
-    // the next round's positions, and its gathers before this round's samples are used
-    float tn, tpn;
-    group_advance<G>(t, step, step, lim, tn, tpn);
-    const float s = vol_finish_fma(F);
-    F = vox_fetch<SM>(V, VR, tn);
-    const float sl0 = dpp_prev(s);
-    const float sl = j == 0 ? sEnd : sl0;
-    sEnd = dpp_last_to_first<G>(s);
-    const bool live = t > tp && (iter < GXY_MAX_MARCH || j == 0);   // (T_0 ends no interval: tp = t)
-    const bool cross = live && ((sl < iso && s >= iso) || (sl > iso && s <= iso));
-    const unsigned cm = group_bits<G>(__builtin_amdgcn_ballot_w64(cross));
-    const int hit = cm ? __builtin_ctz(cm) : G;
-    nsamp += (live && j <= hit) ? 1u : 0u;
-    if (cm) {
-      if (j == hit) {
-        const float tHit = tp + (((iso - sl) / (s - sl)) * (t - tp));
-        gptr(R.t)[i] = tHit + 0.001f;
-        gptr(R.term)[i] = RAY_SURFACE;
-      }
-      break;
-    }
-    // lane 0's next position is the one after this round's last
-    if (!(group_bits<G>(__builtin_amdgcn_ballot_w64(tn > tpn)) & 1u)) {
-      if (j == G - 1) {
-        gptr(R.t)[i] = go0 ? t : tEntry + step;
-        gptr(R.term)[i] = RAY_BOUNDARY;
-      }
-      break;
-    }
-    if (iter >= GXY_MAX_MARCH) {
-      if (j == 1) {
-        gptr(R.t)[i] = t;
-        gptr(R.term)[i] = RAY_BOUNDARY;
-      }
-      break;
-    }
-    t = tn;
-    tp = tpn;
-  }
-  return nsamp;
-}
-
 // the value of lane k of the group, in all its lanes
 template <int G>
 __device__ __forceinline__ float dpp_bcast(float v, int k) {
@@ -150,6 +79,191 @@ __device__ __forceinline__ float dpp_bcast(float v, int k) {
   GXY_BC(8) GXY_BC(9) GXY_BC(10) GXY_BC(11) GXY_BC(12) GXY_BC(13) GXY_BC(14) GXY_BC(15)
 #undef GXY_BC
   return __int_as_float(r);
+}
+
+// One march of SamplerTraceRays through one volume with G lanes per ray: from t
+// = rt (or the box's entry) to the next crossing of the first isovalue, or out.
+// Position T_0 is the entry point and T_k+1 = min(T_k + step, tExit); the march
+// ends where that no longer advances.  tBox, tExit: the box clip of the ray; rt:
+// its t before and after (the crossing + 0.001, or where it left), in all lanes
+// of the group, as is the returned flag of a crossing.  nsamp: this lane's
+// samples.
+template <int G, int SM>
+__device__ __forceinline__ bool sample_segment(const TraceParams &P, const VoxRay &VR, float tBox, float tExit,
+                                               float &rt, unsigned &nsamp) {
+  const int j = group_lane<G>();
+  const DVolume &V = P.vv[0].vol;
+  float tEntry = tBox;
+  if (tEntry < rt) tEntry = rt;
+  const float step = P.step, iso = P.vv[0].iso[0];
+  // the first step is not cut at the exit: a ray whose first step leaves takes
+  // no step at all (its chain stays at the entry)
+  const bool go0 = tEntry + step <= tExit;
+  const float lim = go0 ? tExit : tEntry;
+  float t = tEntry, tp = tEntry;
+#pragma unroll
+  for (int k = 1; k < G; k++)
+    if (k <= j) {
+      tp = t;
+      t += step;
+    }
+  t = __builtin_fminf(t, lim);
+  tp = __builtin_fminf(tp, lim);
+  VFetch F = vox_fetch<SM>(V, VR, t);
+  float sEnd = 0.f;   // lane 0: the last lane's sample of the round before
+  nsamp += j == 0 ? 1u : 0u;
+  // (round `iter` holds positions iter .. iter + G - 1; at most GXY_MAX_MARCH
+  // samples after the first, a multiple of G)
+  for (int iter = 0;; iter += G) {
+    // the next round's positions, and its gathers before this round's samples are used
+    float tn, tpn;
+    group_advance<G>(t, step, step, lim, tn, tpn);
+    const float s = vol_finish_fma(F);
+    F = vox_fetch<SM>(V, VR, tn);
+    const float sl0 = dpp_prev(s);
+    const float sl = j == 0 ? sEnd : sl0;
+    sEnd = dpp_last_to_first<G>(s);
+    const bool live = t > tp && (iter < GXY_MAX_MARCH || j == 0);   // (T_0 ends no interval: tp = t)
+    const bool cross = live && ((sl < iso && s >= iso) || (sl > iso && s <= iso));
+    const unsigned cm = group_bits<G>(__builtin_amdgcn_ballot_w64(cross));
+    const int hit = cm ? __builtin_ctz(cm) : G;
+    nsamp += (live && j <= hit) ? 1u : 0u;
+    if (cm) {
+      const float tHit = tp + (((iso - sl) / (s - sl)) * (t - tp));
+      rt = __shfl(tHit, ((threadIdx.x & 63) & ~(G - 1)) + hit, 64) + 0.001f;
+      return true;
+    }
+    // lane 0's next position is the one after this round's last
+    if (!(group_bits<G>(__builtin_amdgcn_ballot_w64(tn > tpn)) & 1u)) {
+      rt = go0 ? dpp_bcast<G>(t, G - 1) : tEntry + step;
+      return false;
+    }
+    if (iter >= GXY_MAX_MARCH) {
+      rt = dpp_bcast<G>(t, 1);
+      return false;
+    }
+    t = tn;
+    tp = tpn;
+  }
+}
+
+// sample_one of one volume with G lanes per ray (every lane of the group calls
+// it for the same ray, the k-th after the uniform `first`).
+template <int G, int SM>
+__device__ __forceinline__ unsigned sample_group(const TraceParams &P, const RayList_ispc &R, const int first,
+                                                 const unsigned k) {
+  const f3 org = ray_org(R, first, k), dir = ray_dir(R, first, k);
+  float rt = gptr(R.t + first)[k];
+  float tBox, tExit;
+  box_clip(org, dir, P.blo, P.bhi, tBox, tExit);
+  unsigned nsamp = 0;
+  const bool hit = sample_segment<G, SM>(P, vox_ray(P.vv[0].vol, org, dir), tBox, tExit, rt, nsamp);
+  if (group_lane<G>() == 0) {
+    gptr(R.t + first)[k] = rt;
+    gptr(R.term + first)[k] = hit ? RAY_SURFACE : RAY_BOUNDARY;
+  }
+  return nsamp;
+}
+
+// The particles of one wave on their way to a list's array: kept in LDS (buf,
+// 64 of them) and appended 64 at a time, so that the waves of a list do not queue
+// on its counter for every crossing.  Every lane of the wave makes each call.
+struct ParticleBuffer {
+  float *buf;   // 3 x 64 floats of the wave
+  int count;    // uniform
+  __device__ __forceinline__ void flush(float *xyz, int *pcount, int pcap) {
+    if (count == 0) return;
+    const int lane = threadIdx.x & 63;
+    int off = 0;
+    if (lane == 0) off = atomicAdd(pcount, count);
+    off = __builtin_amdgcn_readfirstlane(off);
+    if (lane < count && off + lane < pcap) {
+      float *p = xyz + 3 * (int64_t)(off + lane);
+      for (int a = 0; a < 3; a++) p[a] = buf[64 * a + lane];
+    }
+    count = 0;
+    wave_lds_sync();
+  }
+  __device__ __forceinline__ void add(bool f, f3 p, float *xyz, int *pcount, int pcap) {
+    const unsigned long long m = __builtin_amdgcn_ballot_w64(f);
+    const int n = __popcll(m);
+    if (n == 0) return;
+    if (count + n > 64) flush(xyz, pcount, pcap);
+    if (f) {
+      const int lane = threadIdx.x & 63;
+      const int k = count + __popcll(m & ((1ull << lane) - 1ull));
+      buf[k] = p.x;
+      buf[64 + k] = p.y;
+      buf[128 + k] = p.z;
+    }
+    count += n;
+    wave_lds_sync();
+  }
+};
+
+// The sampler loop without re-queueing for `count` rays after `first` (uniform),
+// by one wave: SamplerTraceRays marches to the next isovalue crossing,
+// Sampler::HandleTerminatedRays appends the particle at o + t*d (t = crossing +
+// 0.001, Sampler.cpp:71-84), and the ray continues from there (the KEEP_HERE
+// re-trace of Renderer.cpp:659-691) until it leaves the volume.  Every segment is
+// one ray pass with the samples of sample_one, so counts and particles equal
+// those of the per-list loop (the particles' order differs).  After max_segments
+// segments a ray is left as a SURFACE ray for the caller to re-queue (its
+// particle not yet emitted).  A group whose ray is done takes the next ray of the
+// range, while the others go on.
+template <int G, int SM>
+__device__ __forceinline__ void sample_range(const TraceParams &P, const RayList_ispc &R, const int first,
+                                             const int count, ParticleBuffer &B, float *xyz, int *pcount, int pcap,
+                                             int max_segments, unsigned long long &samples,
+                                             unsigned long long &passes) {
+  const int lane = threadIdx.x & 63, j = group_lane<G>();
+  const unsigned long long heads = G == 2 ? 0x5555555555555555ull : G == 4 ? 0x1111111111111111ull
+                                   : G == 8 ? 0x0101010101010101ull : 0x0001000100010001ull;
+  int next = 0;            // uniform: rays handed out
+  bool busy = false;
+  unsigned k = 0, nsamp = 0;
+  int segs = 0;
+  f3 org = mk3(0.f, 0.f, 0.f), dir = org;   // dir as stored (the particle's), not the march's
+  VoxRay VR = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  float rt = 0.f, tBox = 0.f, tExit = 0.f;
+  for (;;) {
+    const unsigned long long idle = __builtin_amdgcn_ballot_w64(!busy) & heads;
+    if (idle && next < count) {
+      const int q = next + __popcll(idle & ((1ull << (lane & ~(G - 1))) - 1ull));
+      if (!busy && q < count) {
+        busy = true;
+        k = (unsigned)q;
+        segs = 0;
+        org = ray_org(R, first, k);
+        const f3 d = ray_dir(R, first, k);
+        dir = mk3(gptr(R.dx + first)[k], gptr(R.dy + first)[k], gptr(R.dz + first)[k]);
+        rt = gptr(R.t + first)[k];
+        box_clip(org, d, P.blo, P.bhi, tBox, tExit);
+        VR = vox_ray(P.vv[0].vol, org, d);
+      }
+      next += __popcll(idle);
+    }
+    if (!__builtin_amdgcn_ballot_w64(busy)) break;
+    bool emit = false;
+    f3 p = org;
+    if (busy) {
+      const bool hit = sample_segment<G, SM>(P, VR, tBox, tExit, rt, nsamp);
+      segs++;
+      passes += j == 0 ? 1u : 0u;
+      if (hit && segs < max_segments) {
+        emit = j == 0;
+        p = mk3(org.x + rt * dir.x, org.y + rt * dir.y, org.z + rt * dir.z);
+      } else {
+        busy = false;
+        if (j == 0) {
+          gptr(R.t + first)[k] = rt;
+          gptr(R.term + first)[k] = hit ? RAY_SURFACE : RAY_BOUNDARY;
+        }
+      }
+    }
+    B.add(emit, p, xyz, pcount, pcap);
+  }
+  samples += nsamp;
 }
 
 // trace_one of one volume without geometry, with G lanes per ray (every lane of

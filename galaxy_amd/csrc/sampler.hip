@@ -28,9 +28,10 @@ __global__ __launch_bounds__(GXY_BLOCK) void k_sampler(TraceParams P, RayList_is
 // lane, 1.05 with eight, 0.97 with sixteen.
 template <int G, int SM>
 __global__ __launch_bounds__(GXY_BLOCK) void k_sampler_group(TraceParams P, RayList_ispc R, int n) {
-  const int i = (int)(blockIdx.x * (GXY_BLOCK / G) + threadIdx.x / G);
+  const int first = (int)(blockIdx.x * (GXY_BLOCK / G));
+  const unsigned k = threadIdx.x / G;
   unsigned long long nsamp = 0;
-  if (i < n) nsamp = sample_group<G, SM>(P, R, i);
+  if ((int)k < n - first) nsamp = sample_group<G, SM>(P, R, first, k);
   if (P.sample_count) wave_add_count(nsamp, P.sample_count);
 }
 
