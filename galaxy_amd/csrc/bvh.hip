@@ -882,6 +882,45 @@ __global__ __launch_bounds__(GXY_BLOCK) void k_sah(const BVHNode *nodes, int nn,
   }
 }
 
+// ------------------------------------------------------------------ structural check
+// One mark per child reference: marks[0 .. nn) of the nodes, then nprim of the
+// primitives.  A child's index has to be larger than its parent's, as both the
+// layout and the collapse number them: with every node but the root marked
+// exactly once, the parent links then descend to node 0, so no node is out of
+// reach of the root.
+__device__ __forceinline__ bool mark_child(int i, int c, int nn, int nprim, int *marks) {
+  if (c >= 0) {
+    if (c <= i || c >= nn) return false;
+    atomicAdd(marks + c, 1);
+    return true;
+  }
+  const int code = ~c, first = code >> 4, cnt = (code & 15) + 1;
+  if (first < 0 || first > nprim - cnt) return false;
+  for (int q = first; q < first + cnt; q++) atomicAdd(marks + nn + q, 1);
+  return true;
+}
+__global__ __launch_bounds__(GXY_BLOCK) void k_mark_binary(const BVHNode *nodes, int nn, int nprim, int *marks,
+                                                           int *bad) {
+  const int i = blockIdx.x * GXY_BLOCK + threadIdx.x;
+  if (i >= nn) return;
+  const int c0 = nodes[i].c0, c1 = nodes[i].c1;
+  bool ok = mark_child(i, c0, nn, nprim, marks);
+  if (!(nn == 1 && c1 == c0)) ok = mark_child(i, c1, nn, nprim, marks) && ok;   // (one primitive: both children are it)
+  if (!ok) atomicOr(bad, 1);
+}
+__global__ __launch_bounds__(GXY_BLOCK) void k_mark_wide(const BVH4Node *nodes, int nn, int nprim, int *marks,
+                                                         int *bad) {
+  const int64_t t = (int64_t)blockIdx.x * GXY_BLOCK + threadIdx.x;
+  const int i = (int)(t >> 2), k = (int)t & 3;
+  if (i >= nn) return;
+  if (!(nodes[i].lox[k] <= nodes[i].hix[k])) return;   // empty slot
+  if (!mark_child(i, nodes[i].child[k], nn, nprim, marks)) atomicOr(bad, 1);
+}
+__global__ __launch_bounds__(GXY_BLOCK) void k_check_marks(const int *marks, int n, int *bad) {
+  const int i = blockIdx.x * GXY_BLOCK + threadIdx.x;
+  if (i < n && marks[i] != (i == 0 ? 0 : 1)) atomicOr(bad, 1);
+}
+
 // ------------------------------------------------------------------ driver
 namespace {
 struct Pool {
@@ -1145,6 +1184,35 @@ hipError_t build_lbvh(const float *boxes_dev, int n, float prim_cost, alloc_fn_t
   out->leaves = 0;
   out->heights = maxh;
   return hipGetLastError();
+}
+
+// Every child index in range, every node of both trees and every primitive
+// reached exactly once from the root?  *ok = 0 when not (or when the marks'
+// memory is not there).  Trees without nodes are not looked at.
+hipError_t check_trees(const BVHNode *nodes, int nn, const BVH4Node *nodes4, int nn4, int nprim, alloc_fn_t alloc,
+                       free_fn_t dfree, int *ok, hipStream_t s) {
+  *ok = 0;
+  Pool P{alloc, dfree, {}};
+  const size_t n2 = nn > 0 ? (size_t)nn + nprim : 0, n4 = nn4 > 0 ? (size_t)nn4 + nprim : 0;
+  if (n2 > INT32_MAX || n4 > INT32_MAX) return hipSuccess;
+  int *marks = (int *)P.get(sizeof(int) * (1 + n2 + n4));   // the verdict, then the marks
+  if (!marks) return hipSuccess;
+  BVH_CHK(hipMemsetAsync(marks, 0, sizeof(int) * (1 + n2 + n4), s));
+  int *m2 = marks + 1, *m4 = m2 + n2;
+  auto grid = [](size_t n) { return dim3((unsigned)((n + GXY_BLOCK - 1) / GXY_BLOCK)); };
+  if (n2) {
+    hipLaunchKernelGGL(k_mark_binary, grid(nn), dim3(GXY_BLOCK), 0, s, nodes, nn, nprim, m2, marks);
+    hipLaunchKernelGGL(k_check_marks, grid(n2), dim3(GXY_BLOCK), 0, s, (const int *)m2, (int)n2, marks);
+  }
+  if (n4) {
+    hipLaunchKernelGGL(k_mark_wide, grid(4 * (size_t)nn4), dim3(GXY_BLOCK), 0, s, nodes4, nn4, nprim, m4, marks);
+    hipLaunchKernelGGL(k_check_marks, grid(n4), dim3(GXY_BLOCK), 0, s, (const int *)m4, (int)n4, marks);
+  }
+  BVH_CHK(hipGetLastError());
+  int bad = 1;
+  BVH_CHK(read_ints(marks, &bad, 1, s));
+  *ok = bad == 0;
+  return hipSuccess;
 }
 
 }  // namespace gxy

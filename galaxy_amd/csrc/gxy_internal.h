@@ -262,5 +262,8 @@ struct BVHBuildResult {
 // prim_cost: SAH cost of one primitive test against one node visit's 1.2
 hipError_t build_lbvh(const float *boxes_dev, int n, float prim_cost, alloc_fn_t alloc, free_fn_t dfree,
                       BVHBuildResult *out, hipStream_t s);
+// Structural check of a built tree and its 4-wide form (bvh.hip)
+hipError_t check_trees(const BVHNode *nodes, int nn, const BVH4Node *nodes4, int nn4, int nprim, alloc_fn_t alloc,
+                       free_fn_t dfree, int *ok, hipStream_t s);
 
 }  // namespace gxy

@@ -1379,7 +1379,9 @@ GXY_EXPORT int gxy_model_add_pathlines(void *model, const float *V, const float 
 }
 
 namespace gxy {
-__global__ void k_tri_boxes(const float *V, const uint32_t *I, int nt, float *boxes) {
+// box, geometry and index of every triangle of one mesh
+__global__ void k_tri_boxes(const float *V, const uint32_t *I, int nt, int geom, float *boxes, int *fgeom,
+                            int *fprim) {
   int p = blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= nt) return;
   float lo[3] = {3e38f, 3e38f, 3e38f}, hi[3] = {-3e38f, -3e38f, -3e38f};
@@ -1391,6 +1393,8 @@ __global__ void k_tri_boxes(const float *V, const uint32_t *I, int nt, float *bo
     }
   }
   for (int a = 0; a < 3; a++) { boxes[6 * (int64_t)p + a] = lo[a]; boxes[6 * (int64_t)p + 3 + a] = hi[a]; }
+  fgeom[p] = geom;
+  fprim[p] = p;
 }
 
 __device__ float sphere_radius_dev(float r0, float r1, float v0, float v1, float dv) {
@@ -1404,7 +1408,7 @@ __device__ float sphere_radius_dev(float r0, float r1, float v0, float v1, float
 }
 
 __global__ void k_sph_boxes(const float *C, const float *D, int n, float r0, float r1, float v0, float v1,
-                            float *boxes, float *radius) {
+                            int geom, float e, float *boxes, float *radius, int *fgeom, int *fprim, float *eps) {
   int p = blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= n) return;
   float r = sphere_radius_dev(r0, r1, v0, v1, D[p]);
@@ -1413,6 +1417,9 @@ __global__ void k_sph_boxes(const float *C, const float *D, int n, float r0, flo
     boxes[6 * (int64_t)p + a] = C[3 * (int64_t)p + a] - r;
     boxes[6 * (int64_t)p + 3 + a] = C[3 * (int64_t)p + a] + r;
   }
+  fgeom[p] = geom;
+  fprim[p] = p;
+  eps[p] = e;
 }
 
 // sorted triangle k <- primitive order[k] of the flat list (geom, prim)
@@ -1445,15 +1452,12 @@ __global__ void k_gather_sph(const int *order, const int *fgeom, const int *fpri
 }
 }  // namespace gxy
 
-// Structural check of a built tree: every child index in range, every inner
-// node and every leaf reached exactly once from the root.  Run for trees of up
-// to GXY_BVH_VALIDATE_MAX nodes (default 4M) before the tree is used.
-// Structural check of a 4-wide tree built on the device: child indices in
+// Structural check of a built tree and of its 4-wide form: child indices in
 // range, every node reached once from the root, every primitive in exactly one
-// leaf.  Run for trees of up to GXY_BVH_VALIDATE_MAX nodes (default 4M).
+// leaf.  Run for trees of up to GXY_BVH_VALIDATE_MAX nodes (default 4M) before
+// the tree is used, on the device (check_trees); a tree that fails there is
+// walked on the host, which names the fault.
 static int validate_bvh4(const BVH4Node *d4, int nn4, int nprim, const char *what) {
-  size_t lim = getenv("GXY_BVH_VALIDATE_MAX") ? (size_t)atol(getenv("GXY_BVH_VALIDATE_MAX")) : (size_t)(4u << 20);
-  if ((size_t)nn4 > lim) return 0;
   std::vector<BVH4Node> n4(nn4);
   HIPCHK(hipMemcpyAsync(n4.data(), d4, sizeof(BVH4Node) * nn4, hipMemcpyDeviceToHost, S()));
   HIPCHK(hipStreamSynchronize(S()));
@@ -1485,8 +1489,6 @@ static int validate_bvh4(const BVH4Node *d4, int nn4, int nprim, const char *wha
 }
 
 static int validate_bvh(const BVHNode *dnodes, int nnodes, int nprim, const char *what) {
-  size_t lim = getenv("GXY_BVH_VALIDATE_MAX") ? (size_t)atol(getenv("GXY_BVH_VALIDATE_MAX")) : (size_t)(4u << 20);
-  if ((size_t)nnodes > lim) return 0;
   std::vector<BVHNode> h(nnodes);
   HIPCHK(hipMemcpyAsync(h.data(), dnodes, sizeof(BVHNode) * nnodes, hipMemcpyDeviceToHost, S()));
   HIPCHK(hipStreamSynchronize(S()));
@@ -1515,6 +1517,19 @@ static int validate_bvh(const BVHNode *dnodes, int nnodes, int nprim, const char
   for (int k = 0; k < nprim; k++)
     if (!seen_prim[k]) return fail("%s BVH: primitive %d unreachable", what, k);
   return 0;
+}
+
+// (the download of both trees, 112 MB for 1M triangles, and the walk took 28 of the
+// 37 ms of a step; the kernels take 0.06 ms)
+static int validate_trees(const BVHBuildResult &B, int nprim, const char *what) {
+  size_t lim = getenv("GXY_BVH_VALIDATE_MAX") ? (size_t)atol(getenv("GXY_BVH_VALIDATE_MAX")) : (size_t)(4u << 20);
+  const int nn = (size_t)B.nnodes > lim ? 0 : B.nnodes, nn4 = (size_t)B.nnodes4 > lim ? 0 : B.nnodes4;
+  if (nn == 0 && nn4 == 0) return 0;
+  int ok = 0;
+  HIPCHK(check_trees(B.nodes, nn, B.nodes4, nn4, nprim, dalloc, dfree, &ok, S()));
+  if (ok) return 0;
+  if (nn && validate_bvh(B.nodes, nn, nprim, what) != 0) return -1;
+  return nn4 ? validate_bvh4(B.nodes4, nn4, nprim, what) : 0;
 }
 
 GXY_EXPORT int gxy_model_commit(void *model) {
@@ -1567,16 +1582,18 @@ GXY_EXPORT int gxy_model_commit(void *model) {
   M->d.ngeom = M->ngeom;
   hipStream_t s = S();
   if (ntri > 0) {
-    std::vector<int> fg(ntri), fp(ntri);
     float *boxes = (float *)dalloc(6 * 4 * (size_t)ntri);
-    if (!boxes) return -1;
+    int *dfg = (int *)dalloc(4 * (size_t)ntri), *dfp = (int *)dalloc(4 * (size_t)ntri);
+    if (!boxes || !dfg || !dfp) {
+      for (void *p : {(void *)boxes, (void *)dfg, (void *)dfp}) dfree(p);
+      return -1;
+    }
     int64_t off = 0;
     for (auto &m : M->meshes) {
-      for (int p = 0; p < m.nt; p++) { fg[off + p] = m.geomID; fp[off + p] = p; }
-      hipLaunchKernelGGL(k_tri_boxes, dim3((m.nt + 255) / 256), dim3(256), 0, s, m.V, m.I, m.nt, boxes + 6 * off);
+      hipLaunchKernelGGL(k_tri_boxes, dim3((m.nt + 255) / 256), dim3(256), 0, s, m.V, m.I, m.nt, m.geomID,
+                         boxes + 6 * off, dfg + off, dfp + off);
       off += m.nt;
     }
-    int *dfg = upload(fg.data(), fg.size()), *dfp = upload(fp.data(), fp.size());
     BVHBuildResult B;
     HIPCHK(build_lbvh(boxes, (int)ntri, G.bvh_cost[0], dalloc, dfree, &B, s));
     float *tverts = (float *)dalloc(9 * 4 * (size_t)ntri);
@@ -1598,31 +1615,30 @@ GXY_EXPORT int gxy_model_commit(void *model) {
     M->tnodes = B.nnodes;
     M->tdepth = B.depth;
     if (B.depth > 60) return fail("triangle BVH depth %d exceeds the traversal stack", B.depth);
-    if (validate_bvh(B.nodes, B.nnodes, (int)ntri, "triangle") != 0) return -1;
     M->owned.push_back(B.nodes4);
-    if (validate_bvh4(B.nodes4, B.nnodes4, (int)ntri, "triangle") != 0) return -1;
+    if (validate_trees(B, (int)ntri, "triangle") != 0) return -1;
     M->d.tnodes4 = B.nodes4;
     M->tdepth4 = B.depth4;
     M->tnodes4 = B.nnodes4;
     M->tsah = B.sah;
   }
   if (nsph > 0) {
-    std::vector<int> fg(nsph), fp(nsph);
-    std::vector<float> feps(nsph);
     float *boxes = (float *)dalloc(6 * 4 * (size_t)nsph);
     float *frad = (float *)dalloc(4 * (size_t)nsph);
     float *fC = (float *)dalloc(12 * (size_t)nsph);
-    if (!boxes || !frad || !fC) return -1;
+    int *dfg = (int *)dalloc(4 * (size_t)nsph), *dfp = (int *)dalloc(4 * (size_t)nsph);
+    float *dfe = (float *)dalloc(4 * (size_t)nsph);
+    if (!boxes || !frad || !fC || !dfg || !dfp || !dfe) {
+      for (void *p : {(void *)boxes, (void *)frad, (void *)fC, (void *)dfg, (void *)dfp, (void *)dfe}) dfree(p);
+      return -1;
+    }
     int64_t off = 0;
     for (auto &p : M->spheres) {
-      for (int k = 0; k < p.n; k++) { fg[off + k] = p.geomID; fp[off + k] = k; feps[off + k] = p.eps; }
       hipLaunchKernelGGL(k_sph_boxes, dim3((p.n + 255) / 256), dim3(256), 0, s, p.C, p.D, p.n, p.r0, p.r1, p.v0,
-                         p.v1, boxes + 6 * off, frad + off);
+                         p.v1, p.geomID, p.eps, boxes + 6 * off, frad + off, dfg + off, dfp + off, dfe + off);
       hipMemcpyAsync(fC + 3 * off, p.C, 12 * (size_t)p.n, hipMemcpyDeviceToDevice, s);
       off += p.n;
     }
-    int *dfg = upload(fg.data(), fg.size()), *dfp = upload(fp.data(), fp.size());
-    float *dfe = upload(feps.data(), feps.size());
     BVHBuildResult B;
     HIPCHK(build_lbvh(boxes, (int)nsph, G.bvh_cost[1], dalloc, dfree, &B, s));
     float *sc = (float *)dalloc(12 * (size_t)nsph), *sr = (float *)dalloc(4 * (size_t)nsph);
@@ -1645,9 +1661,8 @@ GXY_EXPORT int gxy_model_commit(void *model) {
     M->snodes = B.nnodes;
     M->sdepth = B.depth;
     if (B.depth > 60) return fail("sphere BVH depth %d exceeds the traversal stack", B.depth);
-    if (validate_bvh(B.nodes, B.nnodes, (int)nsph, "sphere") != 0) return -1;
     M->owned.push_back(B.nodes4);
-    if (validate_bvh4(B.nodes4, B.nnodes4, (int)nsph, "sphere") != 0) return -1;
+    if (validate_trees(B, (int)nsph, "sphere") != 0) return -1;
     M->d.snodes4 = B.nodes4;
     M->sdepth4 = B.depth4;
     M->snodes4 = B.nnodes4;
@@ -1712,9 +1727,8 @@ GXY_EXPORT int gxy_model_commit(void *model) {
     M->cnodes = B.nnodes;
     M->cdepth = B.depth;
     if (B.depth > 60) return fail("curve BVH depth %d exceeds the traversal stack", B.depth);
-    if (validate_bvh(B.nodes, B.nnodes, (int)ncur, "curve") != 0) return -1;
     M->owned.push_back(B.nodes4);
-    if (validate_bvh4(B.nodes4, B.nnodes4, (int)ncur, "curve") != 0) return -1;
+    if (validate_trees(B, (int)ncur, "curve") != 0) return -1;
     M->d.cnodes4 = B.nodes4;
     M->cdepth4 = B.depth4;
     M->cnodes4 = B.nnodes4;
