@@ -10,25 +10,29 @@
 // 3. Karras topology (HPG 2012): one work-item per inner node finds its key
 //    range and split with the delta() prefix length (equal codes broken by
 //    index);
-// 4. bottom-up refit, one launch per depth (depths by pointer jumping over the
-//    parent links, then a counting sort of the inner nodes by depth): child
-//    boxes, primitive counts, heights, and the SAH cost of every subtree both
-//    as built and with the cheaper of leaf or node at each subtree that fits a
-//    leaf.  Kernel boundaries order the levels, so no work-item waits on
-//    another's stores;
-// 5. treelet restructuring (Karras and Aila, "Fast Parallel Construction of
+// 4. treelet restructuring (Karras and Aila, "Fast Parallel Construction of
 //    High-Quality Bounding Volume Hierarchies", HPG 2013): every node with at
 //    least gamma primitives below it roots a treelet of 7 leaves, grown from its
 //    two children by opening the inner leaf of largest surface area; the
 //    SAH-optimal binary tree over those 7 leaves (dynamic programming over the
 //    127 subsets, leaf option included) replaces the treelet when it is
-//    cheaper, reusing its inner nodes.  Nodes are processed by height, lowest
-//    first (one launch per height; treelets of one height are disjoint), three
-//    rounds with gamma = 7, 14, 28;
+//    cheaper, reusing its inner nodes.  Nodes are processed by depth, deepest
+//    first (one launch per depth; treelets of one depth are disjoint, and a
+//    treelet needs the ones below it only, so the tree is that of any bottom-up
+//    order), three rounds with gamma = 7, 14, 28.  The launches refresh primitive
+//    counts and SAH costs as they go and form the boxes in the first round.
+//    Depths come from pointer jumping over the parent links and a counting sort
+//    of the inner nodes by depth.  Kernel boundaries order the levels, so no
+//    work-item waits on another's stores;
+// 5. bottom-up refit, one launch per depth: child boxes, primitive counts, and
+//    the SAH cost with the cheaper of leaf or node at each subtree that fits a
+//    leaf;
 // 6. layout, top-down in breadth-first frontiers: a subtree whose SAH cost is
 //    lower as one leaf (at most GXY_BVH_LEAF primitives) becomes a leaf, inner
 //    nodes are renumbered (root 0, the inner children of a node adjacent) and
-//    the primitives reordered so that every leaf covers a contiguous range;
+//    the primitives reordered so that every leaf covers a contiguous range.  The
+//    frontiers' sizes stay on the device: one launch per depth of the tree, no
+//    wait in between;
 // 7. 4-wide collapse, top-down in frontiers: a node takes its two children and
 //    opens the inner child of largest surface area until it holds four.
 // Node layout: BVHNode (both child boxes, 64 B) and BVH4Node (128 B); child
@@ -269,28 +273,24 @@ __global__ __launch_bounds__(GXY_BLOCK) void k_karras(const uint64_t *keys, int 
 }
 
 // ------------------------------------------------------------------ refit
-// Per inner node: cnt (primitives below), cost (SAH cost as built), costc
-// (SAH cost with each subtree of <= GXY_BVH_LEAF primitives made a leaf where
-// that is cheaper), leaf (1: costc chose a leaf here), height (1 = both
-// children are leaves).  Costs are in units of half surface area.
+// Per inner node: cnt (primitives below), costc (SAH cost with each subtree of
+// <= GXY_BVH_LEAF primitives made a leaf where that is cheaper), leaf (1: costc
+// chose a leaf here).  Costs are in units of half surface area.
 struct BuildArrays {
   int *cnt;
-  float *cost, *costc;
-  int *leaf, *height;
+  float *costc;
+  int *leaf;
   float ct;   // SAH cost of one primitive test
 };
 
 __device__ __forceinline__ void child_totals(const BuildArrays &A, int code, const float lo[3], const float hi[3],
-                                             int &c, float &cost, float &costc, int &h) {
+                                             int &c, float &costc) {
   if (code >= 0) {
     c = A.cnt[code];
-    cost = A.cost[code];
     costc = A.costc[code];
-    h = A.height[code];
   } else {
     c = 1;
-    cost = costc = A.ct * half_area(lo, hi);
-    h = 0;
+    costc = A.ct * half_area(lo, hi);
   }
 }
 
@@ -378,6 +378,22 @@ __global__ __launch_bounds__(GXY_BLOCK) void k_level_scatter(const int *key, int
   }
 }
 
+// The box of node p's slot `slot` from what is below it: an inner child's own
+// two boxes, or the primitive's.
+__device__ __forceinline__ void child_box(const float *boxes, const int *order, const BVHNode *nodes, int code,
+                                          float lo[3], float hi[3]) {
+  if (code >= 0) {
+    const BVHNode *ch = nodes + code;
+    for (int a = 0; a < 3; a++) {
+      lo[a] = fminf(ch->lo0[a], ch->lo1[a]);
+      hi[a] = fmaxf(ch->hi0[a], ch->hi1[a]);
+    }
+  } else {
+    const float *pb = boxes + 6 * (int64_t)order[(~code) >> 4];
+    for (int a = 0; a < 3; a++) { lo[a] = pb[a]; hi[a] = pb[3 + a]; }
+  }
+}
+
 // Refit of the inner nodes of one depth (every deeper node done by earlier
 // launches): the children's boxes go into this node's slots, and the totals
 // of its subtree are formed from the children's.
@@ -387,21 +403,12 @@ __global__ __launch_bounds__(GXY_BLOCK) void k_refit_level(const float *boxes, c
   if (i >= count) return;
   const int p = list[i];
   BVHNode *nd = nodes + p;
-  float l[2][3], h[2][3], s[2], q[2];
-  int c[2], g[2];
+  float l[2][3], h[2][3], q[2];
+  int c[2];
   for (int slot = 0; slot < 2; slot++) {
     const int code = slot ? nd->c1 : nd->c0;
-    if (code >= 0) {
-      const BVHNode *ch = nodes + code;
-      for (int a = 0; a < 3; a++) {
-        l[slot][a] = fminf(ch->lo0[a], ch->lo1[a]);
-        h[slot][a] = fmaxf(ch->hi0[a], ch->hi1[a]);
-      }
-    } else {
-      const float *pb = boxes + 6 * (int64_t)order[(~code) >> 4];
-      for (int a = 0; a < 3; a++) { l[slot][a] = pb[a]; h[slot][a] = pb[3 + a]; }
-    }
-    child_totals(A, code, l[slot], h[slot], c[slot], s[slot], q[slot], g[slot]);
+    child_box(boxes, order, nodes, code, l[slot], h[slot]);
+    child_totals(A, code, l[slot], h[slot], c[slot], q[slot]);
   }
   float lo[3], hi[3];
   for (int a = 0; a < 3; a++) {
@@ -412,14 +419,11 @@ __global__ __launch_bounds__(GXY_BLOCK) void k_refit_level(const float *boxes, c
   }
   const float ar = half_area(lo, hi);
   const int cc = c[0] + c[1];
-  const float cost = BVH_CI * ar + s[0] + s[1];
   const float inner = BVH_CI * ar + q[0] + q[1], asleaf = A.ct * ar * (float)cc;
   const bool lf = p != 0 && cc <= GXY_BVH_LEAF && asleaf <= inner;
   A.cnt[p] = cc;
-  A.cost[p] = cost;
   A.costc[p] = lf ? asleaf : inner;
   A.leaf[p] = lf ? 1 : 0;
-  A.height[p] = max(g[0], g[1]) + 1;
 }
 
 // ------------------------------------------------------------------ treelets
@@ -625,28 +629,28 @@ __device__ __forceinline__ float treelet(BVHNode *nodes, int *parent, const Buil
     if (lane == (s & 63)) {
       const float v = sc[s];
       A.cnt[node] = s >= 64 ? c1 : c0;
-      A.cost[node] = v;
       A.costc[node] = v;
-      A.leaf[node] = 0;
     }
   }
   return best;
 }
 
-// The inner nodes of one height: refresh each node's totals from its children
-// (final: lower heights ran before), and restructure its treelet when it has
-// at least gamma primitives below it.  What a node reads lies below it and no
-// other node of its height writes there.  A wave takes `per` nodes: a lane each
-// for the totals, then all lanes together for one treelet after the other.
+// The inner nodes of one depth: refresh each node's totals from its children
+// (final: deeper nodes ran before), and restructure its treelet when it has at
+// least gamma primitives below it.  What a node reads lies below it and no other
+// node of its depth writes there.  A wave takes `per` nodes: a lane each for the
+// totals, then all lanes together for one treelet after the other.  FIT (the
+// first round): the nodes' boxes are not there yet and come from the children.
 //
 // The search over the 127 subsets (966 pairs of LDS reads) and the treelet's
 // growth (five dependent node reads) are a serial chain: with one work-item per
-// treelet a launch took its 124 us however few nodes the height had, 110 launches
-// 13.7 ms of a build over 1M triangles.  With a wave per treelet: 21 us a launch,
-// 2.3 ms (64 VGPRs, 8 waves per SIMD).
+// treelet a launch took its 124 us however few nodes it had, 110 launches
+// 13.7 ms of a build over 1M triangles.  With a wave per treelet: 33 us a launch of the
+// first round (boxes included), 18 us of the others, 2.5 ms (64 VGPRs, 8 waves per SIMD).
+template <bool FIT>
 __global__ __launch_bounds__(64 * TWAVES) __attribute__((amdgpu_waves_per_eu(8, 8)))
-void k_treelet_level(const int *list, int count, int per, BVHNode *nodes, int *parent, int ni, BuildArrays A,
-                     int gamma) {
+void k_treelet_level(const float *boxes, const int *order, const int *list, int count, int per, BVHNode *nodes,
+                     int *parent, int ni, BuildArrays A, int gamma) {
   __shared__ float s_cost[TWAVES][TLS];
   __shared__ unsigned char s_split[TWAVES][TLS];
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
@@ -656,14 +660,24 @@ void k_treelet_level(const int *list, int count, int per, BVHNode *nodes, int *p
   float cost = 0.f;
   if (have) {
     p = list[i];
-    const BVHNode *nd = nodes + p;
+    BVHNode *nd = nodes + p;
+    const int k0 = nd->c0, k1 = nd->c1;
     float l0[3], h0[3], l1[3], h1[3];
-    slot_box(nd, 0, l0, h0);
-    slot_box(nd, 1, l1, h1);
-    int n0, n1, g0, g1;
-    float s0, s1, q0, q1;
-    child_totals(A, nd->c0, l0, h0, n0, s0, q0, g0);
-    child_totals(A, nd->c1, l1, h1, n1, s1, q1, g1);
+    if (FIT) {
+      child_box(boxes, order, nodes, k0, l0, h0);
+      child_box(boxes, order, nodes, k1, l1, h1);
+      for (int a = 0; a < 3; a++) {
+        nd->lo0[a] = l0[a]; nd->hi0[a] = h0[a];
+        nd->lo1[a] = l1[a]; nd->hi1[a] = h1[a];
+      }
+    } else {
+      slot_box(nd, 0, l0, h0);
+      slot_box(nd, 1, l1, h1);
+    }
+    int n0, n1;
+    float q0, q1;
+    child_totals(A, k0, l0, h0, n0, q0);
+    child_totals(A, k1, l1, h1, n1, q1);
     float lo[3], hi[3];
     for (int a = 0; a < 3; a++) { lo[a] = fminf(l0[a], l1[a]); hi[a] = fmaxf(h0[a], h1[a]); }
     const float ar = half_area(lo, hi);
@@ -671,6 +685,7 @@ void k_treelet_level(const int *list, int count, int per, BVHNode *nodes, int *p
     cost = BVH_CI * ar + q0 + q1;
     if (c <= GXY_BVH_LEAF && p != 0) cost = fminf(cost, A.ct * ar * (float)c);
   }
+  if (FIT) tl_sync();   // the boxes a lane has just stored are read by the lanes that grow the treelet
   unsigned long long todo = __ballot(have && c >= gamma);
   while (todo) {
     const int t = __ffsll((long long)todo) - 1;
@@ -685,10 +700,43 @@ void k_treelet_level(const int *list, int count, int per, BVHNode *nodes, int *p
 }
 
 // ------------------------------------------------------------------ layout
-// A frontier entry: old inner node, new node index, first primitive.
+// A frontier entry: old inner node, first primitive.  Entry k of level L has the
+// node index base[L] + k.  Levels[0 .. GXY_BVH_MAXH] holds the levels' entry
+// counts, Levels[GXY_BVH_MAXH + 1 ...] their bases: a launch reads its own count
+// and adds up the next one's, so no level waits for the host.
 struct LayEnt {
-  int old, idx, first;
+  int old, first;
 };
+#define LEVELS (GXY_BVH_MAXH + 1)
+#define LV_BLOCK 1024
+
+// Positions for `want` (0 .. 4) entries per work-item at the end of the next
+// level: one atomic per workgroup (a level's counter is one address; an atomic
+// on it per wave took as long as the level's work).
+__device__ __forceinline__ int level_reserve(int want, int *next_count) {
+  __shared__ int s_w[LV_BLOCK / 64], s_base;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+  int at = 0, sum = 0;
+#pragma unroll
+  for (int k = 0; k < 4; k++) {
+    const unsigned long long m = __ballot(want > k);
+    at += __popcll(m & rs_lanemask_lt());
+    sum += __popcll(m);
+  }
+  if (lane == 0) s_w[w] = sum;
+  __syncthreads();
+  if (threadIdx.x == 0) {
+    int t = 0;
+    for (int q = 0; q < LV_BLOCK / 64; q++) {
+      const int v = s_w[q];
+      s_w[q] = t;
+      t += v;
+    }
+    s_base = t ? atomicAdd(next_count, t) : 0;
+  }
+  __syncthreads();
+  return s_base + s_w[w] + at;
+}
 
 // Primitives of the subtree under code in depth-first order (at most
 // GXY_BVH_LEAF of them, so at most GXY_BVH_LEAF - 1 inner nodes).
@@ -711,31 +759,34 @@ __device__ int subtree_prims(const BVHNode *nodes, int code, int *out) {
   return n;
 }
 
-__global__ __launch_bounds__(GXY_BLOCK) void k_layout(const LayEnt *fr, int count, const BVHNode *nodes, int n,
-                                                      const int *cnt, const int *leaf, const int *order,
-                                                      BVHNode *out, int *neworder, int *ctr, LayEnt *next,
-                                                      int *bad, int cap) {
-  const int i = blockIdx.x * GXY_BLOCK + threadIdx.x;
-  if (i >= count) return;
-  const LayEnt e = fr[i];
-  if (e.idx < 0 || e.idx >= cap) {   // more inner nodes than the tree has: malformed
+__global__ __launch_bounds__(LV_BLOCK) void k_layout(const LayEnt *fr, int level, int *lv, const BVHNode *nodes, int n,
+                                                     const int *cnt, const int *leaf, const int *order, BVHNode *out,
+                                                     int *neworder, LayEnt *next, int *bad, int cap) {
+  const int count = lv[level], base = lv[LEVELS + level], nbase = base + count;
+  if ((int64_t)blockIdx.x * LV_BLOCK >= count) return;   // (blocks of a level smaller than its bound)
+  const int i = blockIdx.x * LV_BLOCK + threadIdx.x;
+  if (i == 0) lv[LEVELS + level + 1] = nbase;
+  const bool have = i < count && nbase <= cap;
+  LayEnt e = {0, 0};
+  BVHNode nd;
+  int cc[2] = {-1, -1}, ninner = 0;
+  bool in[2] = {false, false};
+  if (have) {
+    e = fr[i];
+    nd = nodes[e.old];
+    cc[0] = nd.c0;
+    cc[1] = nd.c1;
+    for (int s = 0; s < 2; s++) {
+      in[s] = cc[s] >= 0 && !leaf[cc[s]];
+      ninner += in[s];
+    }
+  }
+  const int nslot = level_reserve(ninner, lv + level + 1);
+  if (i < count && (!have || nbase + nslot + ninner > cap)) {   // more inner nodes than the tree has: malformed
     atomicAdd(bad, 1);
     return;
   }
-  const BVHNode nd = nodes[e.old];
-  const int cc[2] = {nd.c0, nd.c1};
-  int ninner = 0;
-  for (int s = 0; s < 2; s++) ninner += (cc[s] >= 0 && !leaf[cc[s]]) ? 1 : 0;
-  int base = 0, nslot = 0;
-  if (ninner) {
-    base = atomicAdd(ctr, ninner);
-    nslot = atomicAdd(ctr + 1, ninner);
-    if (nslot + ninner > cap) {
-      atomicAdd(bad, 1);
-      return;
-    }
-  }
-  BVHNode o = nd;
+  if (!have) return;
   int first = e.first, k = 0;
   for (int s = 0; s < 2; s++) {
     const int c = cc[s];
@@ -745,7 +796,7 @@ __global__ __launch_bounds__(GXY_BLOCK) void k_layout(const LayEnt *fr, int coun
       else atomicAdd(bad, 1);
       code = leaf_code_n(first, 1);
       first += 1;
-    } else if (leaf[c]) {
+    } else if (!in[s]) {
       int prims[GXY_BVH_LEAF];
       const int m = subtree_prims(nodes, c, prims);
       if (m < 1 || m > GXY_BVH_LEAF || first + m > n) {
@@ -757,36 +808,38 @@ __global__ __launch_bounds__(GXY_BLOCK) void k_layout(const LayEnt *fr, int coun
         first += m;
       }
     } else {
-      const int idx = base + k;
-      next[nslot + k] = {c, idx, first};
+      next[nslot + k] = {c, first};
+      code = nbase + nslot + k;
       k++;
-      code = idx;
       first += cnt[c];
     }
-    if (s == 0) o.c0 = code;
-    else o.c1 = code;
+    if (s == 0) nd.c0 = code;
+    else nd.c1 = code;
   }
-  o.pad_[0] = o.pad_[1] = 0;
-  out[e.idx] = o;
+  nd.pad_[0] = nd.pad_[1] = 0;
+  out[base + i] = nd;
 }
 
 // ------------------------------------------------------------------ 4-wide collapse
-struct WideEnt {
-  int bin, idx;
-};
+// level 0: one entry (ints zeros), index 0
+__global__ __launch_bounds__(LV_BLOCK) void k_levels_init(int *lv, int *bad, int *entry, int ints) {
+  for (int k = threadIdx.x; k < 2 * LEVELS; k += LV_BLOCK) lv[k] = k == 0 ? 1 : 0;
+  if ((int)threadIdx.x < ints) entry[threadIdx.x] = 0;
+  if (threadIdx.x == 0) *bad = 0;
+}
 
-__global__ __launch_bounds__(GXY_BLOCK) void k_wide(const WideEnt *fr, int count, const BVHNode *nodes,
-                                                    BVH4Node *out, int *ctr, WideEnt *next, int cap, int *bad) {
-  const int i = blockIdx.x * GXY_BLOCK + threadIdx.x;
-  if (i >= count) return;
-  const WideEnt e = fr[i];
-  if (e.idx < 0 || e.idx >= cap || e.bin < 0 || e.bin >= cap) {
-    atomicAdd(bad, 1);
-    return;
-  }
+// (frontier entries: binary nodes)
+__global__ __launch_bounds__(LV_BLOCK) void k_wide(const int *fr, int level, int *lv, const BVHNode *nodes,
+                                                   BVH4Node *out, int *next, int cap, int *bad) {
+  const int count = lv[level], base = lv[LEVELS + level], nbase = base + count;
+  if ((int64_t)blockIdx.x * LV_BLOCK >= count) return;
+  const int i = blockIdx.x * LV_BLOCK + threadIdx.x;
+  if (i == 0) lv[LEVELS + level + 1] = nbase;
+  const int bin = i < count && nbase <= cap ? fr[i] : -1;
+  const bool have = bin >= 0 && bin < cap;
   int code[4];
   float lo[4][3], hi[4][3];
-  const BVHNode b = nodes[e.bin];
+  const BVHNode b = nodes[have ? bin : 0];
   code[0] = b.c0;
   code[1] = b.c1;
   for (int a = 0; a < 3; a++) { lo[0][a] = b.lo0[a]; hi[0][a] = b.hi0[a]; lo[1][a] = b.lo1[a]; hi[1][a] = b.hi1[a]; }
@@ -824,15 +877,12 @@ __global__ __launch_bounds__(GXY_BLOCK) void k_wide(const WideEnt *fr, int count
 #pragma unroll
   for (int j = 0; j < 4; j++)
     if (j < m && code[j] >= 0) ninner++;
-  int base = 0, nslot = 0;
-  if (ninner) {
-    base = atomicAdd(ctr, ninner);
-    nslot = atomicAdd(ctr + 1, ninner);
-    if (nslot + ninner > cap) {
-      atomicAdd(bad, 1);
-      return;
-    }
+  const int nslot = level_reserve(have ? ninner : 0, lv + level + 1);
+  if (i < count && (!have || nbase + nslot + ninner > cap)) {
+    atomicAdd(bad, 1);
+    return;
   }
+  if (!have) return;
   BVH4Node o;
   int k = 0;
 #pragma unroll
@@ -841,8 +891,8 @@ __global__ __launch_bounds__(GXY_BLOCK) void k_wide(const WideEnt *fr, int count
       o.lox[j] = lo[j][0]; o.loy[j] = lo[j][1]; o.loz[j] = lo[j][2];
       o.hix[j] = hi[j][0]; o.hiy[j] = hi[j][1]; o.hiz[j] = hi[j][2];
       if (code[j] >= 0) {
-        next[nslot + k] = {code[j], base + k};
-        o.child[j] = base + k;
+        next[nslot + k] = code[j];
+        o.child[j] = nbase + nslot + k;
         k++;
       } else {
         o.child[j] = code[j];
@@ -854,7 +904,7 @@ __global__ __launch_bounds__(GXY_BLOCK) void k_wide(const WideEnt *fr, int count
     }
     o.pad_[j] = 0;
   }
-  out[e.idx] = o;
+  out[base + i] = o;
 }
 
 // ------------------------------------------------------------------ SAH of the final tree
@@ -969,11 +1019,11 @@ static hipError_t sort_by_level(const int *key, int n, int *hh, int *cnt, int *s
   return hipGetLastError();
 }
 
-// Bottom-up refit of the ni inner nodes, one launch per depth, deepest
-// first; t0..t3 are ni ints each of scratch, list ni ints.
-static hipError_t refit_levels(const float *boxes, const int *order, int ni, BVHNode *nodes, const int *parent,
-                               const BuildArrays &A, int *t0, int *t1, int *t2, int *t3, int *hh, int *list,
-                               hipStream_t s) {
+// The ni inner nodes sorted by depth (cnt and start of each depth on the host,
+// the list on the device) and the number of depths; t0..t3 are ni ints each of
+// scratch.
+static hipError_t sort_by_depth(int ni, const int *parent, int *t0, int *t1, int *t2, int *t3, int *hh, int *cnt,
+                                int *start, int *list, int *depths, hipStream_t s) {
   const dim3 grid((ni + GXY_BLOCK - 1) / GXY_BLOCK);
   hipLaunchKernelGGL(k_depth_init, grid, dim3(GXY_BLOCK), 0, s, parent, ni, t0, t1);
   int *anc = t0, *dep = t1, *anc2 = t2, *dep2 = t3;
@@ -982,13 +1032,11 @@ static hipError_t refit_levels(const float *boxes, const int *order, int ni, BVH
     int *t = anc; anc = anc2; anc2 = t;
     t = dep; dep = dep2; dep2 = t;
   }
-  int cnt[GXY_BVH_MAXH], start[GXY_BVH_MAXH + 1];
   BVH_CHK(sort_by_level(dep, ni, hh, cnt, start, list, s));
-  for (int d = GXY_BVH_MAXH - 2; d >= 0; d--)
-    if (cnt[d] > 0)
-      hipLaunchKernelGGL(k_refit_level, dim3((cnt[d] + GXY_BLOCK - 1) / GXY_BLOCK), dim3(GXY_BLOCK), 0, s, boxes,
-                         order, nodes, (const int *)(list + start[d]), cnt[d], A);
-  return hipGetLastError();
+  *depths = 0;
+  for (int d = 0; d < GXY_BVH_MAXH; d++)
+    if (cnt[d] > 0) *depths = d + 1;
+  return hipSuccess;
 }
 
 hipError_t build_lbvh(const float *boxes_dev, int n, float prim_cost, alloc_fn_t alloc, free_fn_t dfree,
@@ -1062,68 +1110,67 @@ hipError_t build_lbvh(const float *boxes_dev, int n, float prim_cost, alloc_fn_t
   BuildArrays A;
   A.ct = prim_cost;
   A.cnt = (int *)P.get(sizeof(int) * (size_t)ni);
-  A.cost = (float *)P.get(sizeof(float) * (size_t)ni);
   A.costc = (float *)P.get(sizeof(float) * (size_t)ni);
   A.leaf = (int *)P.get(sizeof(int) * (size_t)ni);
-  A.height = (int *)P.get(sizeof(int) * (size_t)ni);
   int *hh = (int *)P.get(sizeof(int) * 2 * GXY_BVH_MAXH);
   int *hlist = (int *)P.get(sizeof(int) * (size_t)ni);
-  if (!nodes || !parent || !t0 || !t1 || !t2 || !t3 || !A.cnt || !A.cost || !A.costc || !A.leaf || !A.height || !hh || !hlist)
+  if (!nodes || !parent || !t0 || !t1 || !t2 || !t3 || !A.cnt || !A.costc || !A.leaf || !hh || !hlist)
     return hipErrorOutOfMemory;
   hipLaunchKernelGGL(k_karras, dim3((ni + GXY_BLOCK - 1) / GXY_BLOCK), dim3(GXY_BLOCK), 0, s, (const uint64_t *)keys,
                      n, nodes, parent);
   P.release(k0);
   P.release(k1);
-  // 4-5: refit, then treelet rounds (each followed by a refit for heights and totals)
-  int maxh = 0;
-  for (int round = 0; round <= 3; round++) {
-    BVH_CHK(refit_levels(boxes_dev, (const int *)order, ni, nodes, (const int *)parent, A, t0, t1, t2, t3, hh, hlist,
-                         s));
-    if (round == 3 || ni < TL) break;
-    // inner nodes by height
-    int hcount[GXY_BVH_MAXH], hstart[GXY_BVH_MAXH + 1];
-    BVH_CHK(sort_by_level((const int *)A.height, ni, hh, hcount, hstart, hlist, s));
+  // 4-5: treelet rounds, then the refit
+  int dcount[GXY_BVH_MAXH], dstart[GXY_BVH_MAXH + 1], depths = 0;
+  for (int round = 0; round < 3 && ni >= TL; round++) {
+    BVH_CHK(sort_by_depth(ni, parent, t0, t1, t2, t3, hh, dcount, dstart, hlist, &depths, s));
+    if (depths > GXY_BVH_MAXH - 2) return hipErrorInvalidValue;
     const int gamma = TL << round;
-    for (int h = 1; h < GXY_BVH_MAXH; h++) {
-      if (hcount[h] == 0) continue;
-      maxh = h > maxh ? h : maxh;
-      // one node per wave while the height leaves waves free, else an equal share of 8192 waves
-      int per = (hcount[h] + 8191) / 8192;
+    for (int d = depths - 1; d >= 0; d--) {
+      if (dcount[d] == 0) continue;
+      // One node per wave up to 65536 nodes, else an equal share: which nodes of a
+      // depth have a treelet is uneven, so far more waves than run at a time (8192)
+      // even it out.  Commit of 1M triangles with 8192 / 16384 / 32768 / 65536 / any
+      // number of waves: 6.58 / 5.48 / 4.99 / 4.81 / 4.94 ms.
+      int per = (dcount[d] + 65535) / 65536;
       per = per < 64 ? per : 64;
-      const int waves = (hcount[h] + per - 1) / per;
-      hipLaunchKernelGGL(k_treelet_level, dim3((waves + TWAVES - 1) / TWAVES), dim3(64 * TWAVES), 0, s,
-                         (const int *)(hlist + hstart[h]), hcount[h], per, nodes, parent, ni, A, gamma);
+      const int waves = (dcount[d] + per - 1) / per;
+      const dim3 grid((waves + TWAVES - 1) / TWAVES), block(64 * TWAVES);
+      if (round == 0)
+        hipLaunchKernelGGL(k_treelet_level<true>, grid, block, 0, s, boxes_dev, (const int *)order,
+                           (const int *)(hlist + dstart[d]), dcount[d], per, nodes, parent, ni, A, gamma);
+      else
+        hipLaunchKernelGGL(k_treelet_level<false>, grid, block, 0, s, boxes_dev, (const int *)order,
+                           (const int *)(hlist + dstart[d]), dcount[d], per, nodes, parent, ni, A, gamma);
     }
     BVH_CHK(hipGetLastError());
   }
+  BVH_CHK(sort_by_depth(ni, parent, t0, t1, t2, t3, hh, dcount, dstart, hlist, &depths, s));
+  for (int d = depths - 1; d >= 0; d--)
+    if (dcount[d] > 0)
+      hipLaunchKernelGGL(k_refit_level, dim3((dcount[d] + GXY_BLOCK - 1) / GXY_BLOCK), dim3(GXY_BLOCK), 0, s, boxes_dev,
+                         (const int *)order, nodes, (const int *)(hlist + dstart[d]), dcount[d], A);
   // 6: layout (leaf collapse, renumbering, primitive order)
   BVHNode *fin = (BVHNode *)P.get(sizeof(BVHNode) * (size_t)ni);
   int *neworder = (int *)P.get(sizeof(int) * (size_t)n);
   LayEnt *fa = (LayEnt *)P.get(sizeof(LayEnt) * (size_t)ni), *fb = (LayEnt *)P.get(sizeof(LayEnt) * (size_t)ni);
-  int *ctr = (int *)P.get(sizeof(int) * 8);
-  if (!fin || !neworder || !fa || !fb || !ctr) return hipErrorOutOfMemory;
-  {
-    const LayEnt root = {0, 0, 0};
-    const int init[8] = {1, 0, 0, 0, 0, 0, 0, 0};   // nodes used, next-frontier entries, malformed leaves
-    BVH_CHK(hipMemcpyAsync(fa, &root, sizeof root, hipMemcpyHostToDevice, s));
-    BVH_CHK(hipMemcpyAsync(ctr, init, sizeof init, hipMemcpyHostToDevice, s));
-  }
-  int count = 1, levels = 0, nn = 1;
-  while (count > 0) {
-    if (++levels > GXY_BVH_MAXH) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_layout, dim3((count + GXY_BLOCK - 1) / GXY_BLOCK), dim3(GXY_BLOCK), 0, s, (const LayEnt *)fa,
-                       count, (const BVHNode *)nodes, n, (const int *)A.cnt, (const int *)A.leaf,
-                       (const int *)order, fin, neworder, ctr, fb, ctr + 2, ni);
-    int c3[3];
-    BVH_CHK(read_ints(ctr, c3, 3, s));
-    if (c3[2] != 0) return hipErrorInvalidValue;
-    nn = c3[0];
-    count = c3[1];
-    BVH_CHK(hipMemsetAsync(ctr + 1, 0, sizeof(int), s));
+  int *lv = (int *)P.get(sizeof(int) * 2 * LEVELS), *bad = (int *)P.get(sizeof(int));
+  if (!fin || !neworder || !fa || !fb || !lv || !bad) return hipErrorOutOfMemory;
+  hipLaunchKernelGGL(k_levels_init, dim3(1), dim3(LV_BLOCK), 0, s, lv, bad, (int *)fa, (int)(sizeof(LayEnt) / 4));
+  // (a level has at most the nodes of its depth)
+  for (int d = 0; d < depths; d++) {
+    hipLaunchKernelGGL(k_layout, dim3((dcount[d] + LV_BLOCK - 1) / LV_BLOCK), dim3(LV_BLOCK), 0, s, (const LayEnt *)fa,
+                       d, lv, (const BVHNode *)nodes, n, (const int *)A.cnt, (const int *)A.leaf, (const int *)order,
+                       fin, neworder, fb, bad, ni);
     LayEnt *t = fa;
     fa = fb;
     fb = t;
   }
+  int hlv[LEVELS], hbad = 0, nn = 0, levels = 0;
+  BVH_CHK(hipMemcpyAsync(&hbad, bad, sizeof hbad, hipMemcpyDeviceToHost, s));
+  BVH_CHK(read_ints(lv, hlv, depths + 1, s));
+  if (hbad != 0 || hlv[depths] != 0) return hipErrorInvalidValue;
+  for (; levels < depths && hlv[levels] > 0; levels++) nn += hlv[levels];
   P.release(nodes);
   P.release(parent);
   P.release(t0);
@@ -1132,29 +1179,30 @@ hipError_t build_lbvh(const float *boxes_dev, int n, float prim_cost, alloc_fn_t
   P.release(t3);
   // 7: 4-wide collapse
   BVH4Node *w4 = (BVH4Node *)P.get(sizeof(BVH4Node) * (size_t)nn);
-  WideEnt *wa = (WideEnt *)P.get(sizeof(WideEnt) * (size_t)nn), *wb = (WideEnt *)P.get(sizeof(WideEnt) * (size_t)nn);
+  int *wa = (int *)P.get(sizeof(int) * (size_t)nn), *wb = (int *)P.get(sizeof(int) * (size_t)nn);
   if (!w4 || !wa || !wb) return hipErrorOutOfMemory;
-  {
-    const WideEnt root = {0, 0};
-    const int init[3] = {1, 0, 0};
-    BVH_CHK(hipMemcpyAsync(wa, &root, sizeof root, hipMemcpyHostToDevice, s));
-    BVH_CHK(hipMemcpyAsync(ctr, init, sizeof init, hipMemcpyHostToDevice, s));
-  }
-  int wcount = 1, wlevels = 0, nn4 = 1;
-  while (wcount > 0) {
-    if (++wlevels > GXY_BVH_MAXH) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(k_wide, dim3((wcount + GXY_BLOCK - 1) / GXY_BLOCK), dim3(GXY_BLOCK), 0, s,
-                       (const WideEnt *)wa, wcount, (const BVHNode *)fin, w4, ctr, wb, nn, ctr + 2);
-    int c2[3];
-    BVH_CHK(read_ints(ctr, c2, 3, s));
-    if (c2[2] != 0) return hipErrorInvalidValue;
-    nn4 = c2[0];
-    wcount = c2[1];
-    BVH_CHK(hipMemsetAsync(ctr + 1, 0, sizeof(int), s));
-    WideEnt *t = wa;
+  hipLaunchKernelGGL(k_levels_init, dim3(1), dim3(LV_BLOCK), 0, s, lv, bad, wa, 1);
+  // (a level has at most four times the nodes of the one above, the tree at most the
+  // binary one's levels; how many is known once a level is empty: looked up every 8)
+  int nn4 = 0, wlevels = 0;
+  int64_t bound = 1;
+  for (int d = 0; d <= levels; d++) {
+    if (d == levels || (d > 0 && d % 8 == 0)) {
+      BVH_CHK(hipMemcpyAsync(&hbad, bad, sizeof hbad, hipMemcpyDeviceToHost, s));
+      BVH_CHK(read_ints(lv, hlv, d + 1, s));
+      if (hbad != 0) return hipErrorInvalidValue;
+      if (hlv[d] == 0) break;
+      if (d == levels) return hipErrorInvalidValue;
+      bound = hlv[d];
+    }
+    hipLaunchKernelGGL(k_wide, dim3((unsigned)((bound + LV_BLOCK - 1) / LV_BLOCK)), dim3(LV_BLOCK), 0, s,
+                       (const int *)wa, d, lv, (const BVHNode *)fin, w4, wb, nn, bad);
+    bound = bound * 4 < nn ? bound * 4 : nn;
+    int *t = wa;
     wa = wb;
     wb = t;
   }
+  for (; wlevels < levels && hlv[wlevels] > 0; wlevels++) nn4 += hlv[wlevels];
   // SAH cost of the final binary tree, relative to the root's surface
   double *acc = (double *)P.get(sizeof(double));
   if (!acc) return hipErrorOutOfMemory;
@@ -1182,7 +1230,6 @@ hipError_t build_lbvh(const float *boxes_dev, int n, float prim_cost, alloc_fn_t
   out->depth4 = wlevels;
   out->sah = ra > 0.0 ? (float)(sah / ra) : 0.f;
   out->leaves = 0;
-  out->heights = maxh;
   return hipGetLastError();
 }
 

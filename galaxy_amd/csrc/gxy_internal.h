@@ -257,7 +257,6 @@ struct BVHBuildResult {
   int nnodes4;
   int depth4;         // levels of 4-wide inner nodes
   int leaves;
-  int heights;        // height of the tree before the last treelet round
 };
 // prim_cost: SAH cost of one primitive test against one node visit's 1.2
 hipError_t build_lbvh(const float *boxes_dev, int n, float prim_cost, alloc_fn_t alloc, free_fn_t dfree,
