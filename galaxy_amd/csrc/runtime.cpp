@@ -3301,11 +3301,18 @@ GXY_EXPORT int gxy_batch_run(void *b, int graph_passes, gxy_batch_stats *st) {
   // capacities for the worst case of pass 0 (every primary ray spawning)
   std::vector<BatchChunk> init;
   long long nprim = 0;
+  // Lists of one dataset next to each other in the queue: its volume or tree then
+  // stays in the last-level cache while its chunks run.  64 lists over 16 datasets
+  // (up to 226 MB each): 12.6 ms in the order of their adding, 11.95 by dataset
+  // (volumes or geometry first, or the largest first: 12.0 to 12.4).
+  std::vector<int> order;
   for (size_t l = 0; l < B->lists.size(); l++)
-    if (B->live[l]) {
-      batch_chunks_of(B, (int)l, init);
-      nprim += B->lists[l].n;
-    }
+    if (B->live[l]) order.push_back((int)l);
+  std::stable_sort(order.begin(), order.end(), [&](int a, int c) { return B->lists[a].ds < B->lists[c].ds; });
+  for (int l : order) {
+    batch_chunks_of(B, l, init);
+    nprim += B->lists[l].n;
+  }
   if (batch_ensure_base(B) != 0) return -1;
   const long long nch = (long long)init.size();
   if (grow((void **)&B->tab[1], &B->tcap[1], nch + 16, sizeof(BatchChunk)) != 0) return -1;
