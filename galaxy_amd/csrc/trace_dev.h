@@ -288,8 +288,8 @@ __device__ __forceinline__ void bvh_walk(const BVHNode *nodes, f3 o, f3 inv, flo
 //   at most 2^-23 |o/d| + 2^-23 |t|, so the near planes are moved towards the
 //   origin and the far planes away from it by 2^-21 |o/d| and the far planes
 //   scaled by 1 + 1.2e-6: a box is only ever entered needlessly, never missed.
-//   An axis whose direction underflows (1/d infinite) gives NaN planes, which
-//   max and min skip;
+//   An axis whose direction underflows (1/d, or 1/d scaled, infinite) gives NaN
+//   planes, which max and min skip;
 // - the near and far planes of an axis are loaded from the lo or hi row by a
 //   per-ray byte offset instead of being selected after the load;
 // - every child is written to the top of the stack and the top moves only for
@@ -305,8 +305,8 @@ __device__ __forceinline__ void bvh4_walk(const BVH4Node *nodes, f3 o, f3 inv, f
   const float ox = o.x * inv.x, oy = o.y * inv.y, oz = o.z * inv.z;
   const float px = PAD * fabsf(ox), py = PAD * fabsf(oy), pz = PAD * fabsf(oz);
   const float nx = -ox - px, ny = -oy - py, nz = -oz - pz;
-  const float fx = px - ox * FS, fy = py - oy * FS, fz = pz - oz * FS;
   const f3 invf = mk3(inv.x * FS, inv.y * FS, inv.z * FS);
+  const float fx = px - o.x * invf.x, fy = py - o.y * invf.y, fz = pz - o.z * invf.z;
   const unsigned bx = inv.x < 0.f ? 48u : 0u, by = inv.y < 0.f ? 64u : 16u, bz = inv.z < 0.f ? 80u : 32u;
   const char *nb = (const char *)gptr(nodes);
   int sp = 0;

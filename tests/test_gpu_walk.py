@@ -129,3 +129,37 @@ def test_mixed_scenes_take_the_same_walks(hip):
         L.gxy_set_bvh_width(2)
         L.gxy_set_geometry_stack(0)
     assert all(np.array_equal(a, b) for a, b in zip(*got))
+
+
+def _closest(hip, B, hr, width, stack):
+    from galaxy_amd import lib as glib
+    L = glib.lib()
+    geom, prim = glib.DeviceArray(4 * hr.n), glib.DeviceArray(4 * hr.n)
+    glib.check(L.gxy_model_set_hit_output(B.vis.model, geom.ptr, prim.ptr))
+    try:
+        glib.check(L.gxy_set_bvh_width(width))
+        glib.check(L.gxy_set_geometry_stack(stack))
+        d = glib.DeviceRays.from_host(hr)
+        assert hip.trace(B.vis, d) == ""
+        return d.download()["t"], geom.to_host(np.int32, hr.n), prim.to_host(np.int32, hr.n)
+    finally:
+        L.gxy_set_bvh_width(2)
+        L.gxy_set_geometry_stack(0)
+        L.gxy_model_set_hit_output(B.vis.model, None, None)
+
+
+@pytest.mark.parametrize("sign", [1, -1])
+def test_directions_whose_reciprocal_nearly_overflows(hip, sign):
+    """1/d is finite, its product with the walk's far-plane factor is not."""
+    B = scenes.build_scene(hip, _scene("blob_spheres"))
+    rng = np.random.default_rng(4)
+    n = 2000
+    o, d = rng.uniform(-0.2, 1.2, (n, 3)), rng.normal(size=(n, 3))
+    least = 1.0 / np.float64(np.finfo(f32).max)          # the smallest d with a finite 1/d
+    for a in range(3):
+        d[a::3, a] = sign * least * rng.uniform(1.0000002, 1.000001, len(d[a::3]))
+    hr = abi.HostRays.from_arrays(o.astype(f32), d.astype(f32), np.zeros(n, f32), np.full(n, 1e30, f32))
+    want, got = _closest(hip, B, hr, 2, 16), _closest(hip, B, hr, 4, 0)
+    assert (want[1] >= 0).sum() > 200
+    for a, b in zip(want, got):
+        assert np.array_equal(a.view(np.int32), b.view(np.int32)), np.nonzero(a != b)[0][:5]
