@@ -900,7 +900,7 @@ __global__ __launch_bounds__(LV_BLOCK) void k_wide(const int *fr, int level, int
     } else {
       o.lox[j] = o.loy[j] = o.loz[j] = __builtin_inff();
       o.hix[j] = o.hiy[j] = o.hiz[j] = -__builtin_inff();
-      o.child[j] = 0x7fffffff;
+      o.child[j] = leaf_code(0);   // (a ray that skips every axis enters this slot too)
     }
     o.pad_[j] = 0;
   }
@@ -1060,7 +1060,7 @@ hipError_t build_lbvh(const float *boxes_dev, int n, float prim_cost, alloc_fn_t
     for (int j = 0; j < 4; j++) {
       w.lox[j] = j ? INFINITY : b[0]; w.loy[j] = j ? INFINITY : b[1]; w.loz[j] = j ? INFINITY : b[2];
       w.hix[j] = j ? -INFINITY : b[3]; w.hiy[j] = j ? -INFINITY : b[4]; w.hiz[j] = j ? -INFINITY : b[5];
-      w.child[j] = j ? 0x7fffffff : leaf_code(0);
+      w.child[j] = leaf_code(0);
       w.pad_[j] = 0;
     }
     out->nodes = (BVHNode *)alloc(sizeof(BVHNode));

@@ -289,7 +289,9 @@ __device__ __forceinline__ void bvh_walk(const BVHNode *nodes, f3 o, f3 inv, flo
 //   origin and the far planes away from it by 2^-21 |o/d| and the far planes
 //   scaled by 1 + 1.2e-6: a box is only ever entered needlessly, never missed.
 //   An axis whose direction underflows (1/d, or 1/d scaled, infinite) gives NaN
-//   planes, which max and min skip;
+//   planes, which max and min skip, and so does one whose o/d overflows.  A ray
+//   that skips all three enters the empty slots of a node as well: their code is
+//   that of the first primitive's leaf, one test more;
 // - the near and far planes of an axis are loaded from the lo or hi row by a
 //   per-ray byte offset instead of being selected after the load;
 // - every child is written to the top of the stack and the top moves only for

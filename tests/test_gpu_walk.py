@@ -163,3 +163,25 @@ def test_directions_whose_reciprocal_nearly_overflows(hip, sign):
     assert (want[1] >= 0).sum() > 200
     for a, b in zip(want, got):
         assert np.array_equal(a.view(np.int32), b.view(np.int32)), np.nonzero(a != b)[0][:5]
+
+
+@pytest.mark.parametrize("spheres", [3, 11, 18, 27, 40])
+def test_rays_that_skip_every_axis_find_all_children(hip, spheres):
+    """Origin over direction overflows on all axes: every slot of a node is
+    entered, the empty ones of nodes with fewer than four children too."""
+    rng = np.random.default_rng(spheres)
+    at, unit = 1e20, 1.4e14                              # (floats near 1e20 are 8.8e12 apart)
+    c = at + unit * rng.integers(0, 5, (spheres, 3))
+    box = ((at - 10 * unit,) * 3, (at + 15 * unit,) * 3)
+    sc = scenes.SceneDesc(local_box=box, global_box=box, spheres=[scenes.SpheresDesc(
+        c.astype(f32), rng.uniform(0, 1, spheres).astype(f32), 0.5 * unit, 0.7 * unit, 0.0, 1.0)])
+    B = scenes.build_scene(hip, sc)
+    n = 1000
+    o = at + unit * rng.integers(-8, 14, (n, 3))
+    d = c[rng.integers(spheres, size=n)] - o + 0.2 * unit * rng.normal(size=(n, 3))
+    d *= 1e-19 / np.linalg.norm(d, axis=1, keepdims=True)
+    hr = abi.HostRays.from_arrays(o.astype(f32), d.astype(f32), np.zeros(n, f32), np.full(n, np.inf, f32))
+    want, got = _closest(hip, B, hr, 2, 16), _closest(hip, B, hr, 4, 0)
+    assert (want[1] >= 0).sum() > 100
+    for a, b in zip(want, got):
+        assert np.array_equal(a.view(np.int32), b.view(np.int32)), np.nonzero(a != b)[0][:5]
