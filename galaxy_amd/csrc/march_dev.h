@@ -133,13 +133,14 @@ __device__ __forceinline__ bool sample_segment(const TraceParams &P, const VoxRa
       rt = __shfl(tHit, ((threadIdx.x & 63) & ~(G - 1)) + hit, 64) + 0.001f;
       return true;
     }
+    // (the last round's position is lane 0's: the march stops at the one after it)
+    if (iter >= GXY_MAX_MARCH) {
+      rt = dpp_bcast<G>(t, 1);
+      return false;
+    }
     // lane 0's next position is the one after this round's last
     if (!(group_bits<G>(__builtin_amdgcn_ballot_w64(tn > tpn)) & 1u)) {
       rt = go0 ? dpp_bcast<G>(t, G - 1) : tEntry + step;
-      return false;
-    }
-    if (iter >= GXY_MAX_MARCH) {
-      rt = dpp_bcast<G>(t, 1);
       return false;
     }
     t = tn;

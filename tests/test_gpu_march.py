@@ -70,6 +70,33 @@ def test_sampler_lanes_take_the_one_ray_march(hip, n, edge, layout, rate):
         assert 0.05 < np.mean(g["term"] == abi.RAY_SURFACE) < 0.95
 
 
+# sixteen lanes per ray and, with rays that miss added, eight
+@pytest.mark.parametrize("extra", [0, 65536])
+def test_sampler_lanes_stop_at_the_step_limit(hip, extra):
+    """Rays that leave the volume a few steps before, at and after the most steps
+    that a march takes (2^20)."""
+    limit = 1 << 20
+    sc = _volume(3, 3, 2.0 / (1.06 * limit))             # (steps of half an edge times the rate)
+    vol = sc.volume_vis[0].volume
+    sc.volume_vis[0].isovalues = np.array([99.0], f32)   # never crossed
+    step = f32(min(vol.spacing)) * f32(vol.sampling_rate)
+    t = np.cumsum(np.full(limit + 40, step), dtype=f32)  # the positions, added up one by one
+    assert t[-1] < 1.0
+    n = 40
+    o = np.full((n, 3), 0.3)
+    o[:, 0] = 1.0 - t[limit - 12:limit + 28].astype(float)
+    d = np.tile([1.0, 0.0, 0.0], (n, 1))
+    o = np.concatenate([o, np.full((extra, 3), 9.0)])
+    d = np.concatenate([d, np.tile([0.0, 0.0, 1.0], (extra, 1))])
+    hr = abi.HostRays.from_arrays(o.astype(f32), d.astype(f32), np.zeros(n + extra, f32), np.full(n + extra, 1e30, f32))
+    g = _sample(hip, sc, 0, hr)
+    sc.volume_vis = [sc.volume_vis[0], scenes.VolumeVisDesc(vol, isovalues=np.array([99.0], f32))]
+    r = _sample(hip, sc, 0, hr)
+    assert len(np.unique(r["t"][:n])) > 10
+    for f in ("t", "term"):
+        assert np.array_equal(g[f].view(np.int32), r[f].view(np.int32)), (f, np.nonzero(g[f] != r[f])[0])
+
+
 def _trace(hip, B, hr, kind):
     from galaxy_amd import lib as glib
     L = glib.lib()
