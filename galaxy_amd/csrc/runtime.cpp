@@ -3123,7 +3123,9 @@ static int batch_dataset_params(BatchObj *B, const Visualization_ispc *vis, floa
   depth = 0;
   if (geometry) {
     ModelObj *M = lookup<ModelObj>(G.models, vis->model);
-    depth = M ? (P.model.wide == 1 ? M->d.depth4 : std::max(M->tdepth, M->sdepth)) : 64;
+    // by the width asked for, also where the 4-wide walk is not taken: the binary
+    // walk's stack goes on in private memory past the entries counted here
+    depth = M ? (G.bvh_width == 4 ? M->d.depth4 : std::max(M->tdepth, M->sdepth)) : 64;
   }
   return 0;
 }

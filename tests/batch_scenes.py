@@ -2,7 +2,7 @@
 volumes over the unit cube (compositing, iso 0.5) and two blob meshes."""
 import numpy as np
 
-from galaxy_amd import scenes, workloads
+from galaxy_amd import abi, scenes, workloads
 
 f32 = np.float32
 
@@ -34,3 +34,27 @@ def dataset_descs():
     out.append(workloads.blob_scene(3000, 7))
     out.append(workloads.blob_scene(20000, 8))
     return out
+
+
+def graded_scene(seed, levels=34, per=12):
+    """Small triangles around the corners of cubes that halve from level to
+    level towards the origin: a deep tree over few primitives."""
+    rng = np.random.default_rng(seed)
+    x = 0.5 ** np.repeat(np.arange(levels), per)
+    c = x[:, None] * rng.choice([0.25, 1.0], (len(x), 3))
+    v = c[:, None] + 0.1 * x[:, None, None] * rng.uniform(-0.5, 0.5, (len(x), 3, 3))
+    box = ((-4.0,) * 3, (4.0,) * 3)
+    return scenes.SceneDesc(meshes=[scenes.MeshDesc(v.reshape(-1, 3).astype(f32),
+                                                    np.arange(3 * len(x), dtype=np.uint32).reshape(-1, 3))],
+                            local_box=box, global_box=box)
+
+
+def rays_at_triangles(sc, n, seed):
+    """Origins around the scene, directions to random triangles of its mesh."""
+    rng = np.random.default_rng(seed)
+    m = sc.meshes[0]
+    c = m.vertices[m.indices].astype(float).mean(1)
+    o = rng.uniform(-1.0, 2.0, (n, 3))
+    d = c[rng.integers(len(c), size=n)] - o
+    d /= np.linalg.norm(d, axis=1, keepdims=True)
+    return abi.HostRays.from_arrays(o.astype(f32), d.astype(f32), np.zeros(n, f32), np.full(n, 1e30, f32))

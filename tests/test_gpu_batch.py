@@ -340,3 +340,38 @@ def test_pending_counts_lists_added_after_a_step(datasets, hip):
     p = B.pending(3 + len(extra))
     assert all(0 <= v <= 50 * 900 for v in p[:3])
     assert [int(p[l]) for l, _ in extra] == [n for _, n in extra]
+
+
+def test_stack_check_counts_the_levels_of_the_width_asked_for(hip):
+    """Width 4 with 32 stack entries takes a tree of 28 4-wide levels (55 binary
+    ones), which the 4-wide walk itself does not, and refuses 24 entries."""
+    from batch_scenes import graded_scene, rays_at_triangles
+    from galaxy_amd import batch as gb
+    from galaxy_amd import lib as glib
+    L = glib.lib()
+    sc = graded_scene(4)
+    built = scenes.build_scene(hip, sc)
+    n, keep, images = 2000, [], []
+    x = np.arange(n, dtype=np.int32)
+    try:
+        for width, stack in ((2, 0), (4, 0), (4, 32), (4, 24)):
+            glib.check(L.gxy_set_bvh_width(width))
+            B = gb.Batch(128)
+            hr = rays_at_triangles(sc, n, 3)
+            hr["x"] = x
+            hr["y"] = 0 * x
+            d = glib.DeviceRays.from_host(hr)
+            l, fb = B.add_render_list(B.add_dataset(built), d, n, 1)
+            B.set_lighting(lights_struct(keep))
+            B.set_config(128, stack, 0, 2)
+            if stack == 24:
+                with pytest.raises(glib.GxyError, match="BVH depth 28 needs"):
+                    B.run(0)
+                continue
+            st = B.run(0)
+            assert st.spawned > 1000
+            images.append(fb.to_host(f32))
+    finally:
+        glib.check(L.gxy_set_bvh_width(2))
+    for im in images[1:]:
+        assert np.abs(im - images[0]).max() <= 1e-5
