@@ -137,16 +137,15 @@ def build_datasets(hip, descs):
 
 
 # candidate launch configurations: (chunk, stack, wpe, blocks per CU, split)
-DEFAULT_CANDIDATES = [(256, 0, 0, 4, 0), (256, 0, 4, 4, 0), (128, 0, 4, 8, 0), (512, 0, 4, 4, 0),
-                      (256, 0, 5, 5, 0), (256, 16, 4, 4, 0), (256, 24, 0, 3, 0), (256, 32, 0, 3, 0),
+DEFAULT_CANDIDATES = [(256, 0, 0, 4, 0), (128, 0, 0, 8, 0), (512, 0, 0, 4, 0), (64, 0, 0, 4, 0),
+                      (256, 16, 0, 4, 0), (256, 24, 0, 3, 0), (256, 32, 0, 3, 0),
                       (256, 0, 0, 4, 1), (256, 0, 5, 4, 1), (256, 24, 5, 4, 1), (128, 0, 5, 8, 1),
-                      (64, 0, 0, 4, 0), (64, 0, 5, 4, 1), (256, 0, 6, 8, 1), (128, 0, 6, 8, 1),
-                      (128, 0, 5, 5, 0), (256, 0, 6, 6, 0)]
+                      (64, 0, 5, 4, 1), (256, 0, 6, 8, 1), (128, 0, 6, 8, 1)]
 
 
 def tune(batch, candidates=None, max_depth=64, graph_passes=2, reps=1):
     """Measures gxy_batch_run under each launch configuration whose traversal
-    stack fits the deepest BVH (stack 0 = private memory, always valid) and
+    stack fits the deepest BVH (stack 0 = the 4-wide walk, always valid) and
     keeps the fastest.  Results do not depend on the configuration; only the
     time does.  Returns (best, [(config, ms), ...])."""
     import time

@@ -223,8 +223,12 @@ __global__ void k_bappend_count(int *ntab, int cap, int n) {
 __global__ void k_bset_count(int *ntab, int v) { *ntab = v; }
 
 // ------------------------------------------------------------------ trace
-template <int STK, int WPE>
-__global__ __launch_bounds__(GXY_BLOCK) __attribute__((amdgpu_waves_per_eu(WPE > 0 ? WPE : 1, 8)))
+// At least 4 waves per SIMD (128 VGPRs): with all kinds inlined the compiler takes
+// 153 (3 waves) by itself, and 64 lists of 16K rays run 13.7 instead of 12.6 ms per
+// flush.  More do not fit: the LDS of a workgroup (36 KB: transfer-function tables,
+// particles, traversal stack) lets four onto a CU.
+template <int STK>
+__global__ __launch_bounds__(GXY_BLOCK) __attribute__((amdgpu_waves_per_eu(4, 8)))
 void k_btrace(BatchArgs A) {
   __shared__ float s_part[BWAVES][3 * 64];
   __shared__ float s_col[BWAVES][1][3 * GXY_TF_MAX];
@@ -701,9 +705,9 @@ __global__ __launch_bounds__(256) void k_fill_f32(float *p, long long n, float v
 __global__ void k_fill_i32_one(int *p, int v) { *p = v; }
 
 // ------------------------------------------------------------------ launchers
-template <int STK, int WPE>
+template <int STK>
 static void btrace_as(const BatchArgs &A, int blocks, hipStream_t s) {
-  hipLaunchKernelGGL((k_btrace<STK, WPE>), dim3(blocks), dim3(GXY_BLOCK), 0, s, A);
+  hipLaunchKernelGGL((k_btrace<STK>), dim3(blocks), dim3(GXY_BLOCK), 0, s, A);
 }
 
 template <int KIND, int STK, int WPE>
@@ -739,15 +743,10 @@ hipError_t launch_batch_pass(const BatchArgs &A, const BatchLaunch &K, hipStream
   const int tb = K.trace_blocks;
   if (K.split && ks && ev) {
     launch_split_trace(A, K, s, ks, ev);
-  } else if (K.stack == 16) btrace_as<16, 4>(A, tb, s);
-  else if (K.stack == 24) btrace_as<24, 4>(A, tb, s);
-  else if (K.stack == 32) btrace_as<32, 4>(A, tb, s);
-  else if (K.wpe == 5) btrace_as<0, 5>(A, tb, s);
-  else if (K.wpe == 6) btrace_as<0, 6>(A, tb, s);
-  // 4 waves per SIMD (128 VGPRs) also when no count is asked for: with all kinds
-  // inlined the compiler takes 153 (3 waves) by itself, and 64 lists of 16K rays
-  // run 13.7 instead of 12.6 ms per flush
-  else btrace_as<0, 4>(A, tb, s);
+  } else if (K.stack == 16) btrace_as<16>(A, tb, s);
+  else if (K.stack == 24) btrace_as<24>(A, tb, s);
+  else if (K.stack == 32) btrace_as<32>(A, tb, s);
+  else btrace_as<0>(A, tb, s);
   hipLaunchKernelGGL(k_bcount, dim3(K.post_blocks), dim3(GXY_BLOCK), 0, s, A);
   hipLaunchKernelGGL(k_bscan_a, dim3(BSCAN_SEG), dim3(256), 0, s, A);
   hipLaunchKernelGGL(k_bscan_b, dim3(1), dim3(BSCAN_SEG), 0, s, A);

@@ -524,9 +524,8 @@ int   gxy_batch_remove_list(void *batch, int list);
 /* Launch configuration: chunk (rays per queue entry, 64..1024), stack (BVH traversal
  * stack: 0 = the 4-wide walk, 16/24/32 = the binary walk, or the 4-wide one with
  * BVH width 4, with that many entries in LDS; must exceed the deepest tree by 2),
- * wpe (waves per SIMD requested: 0, 4, 5 or 6; the fused kernel takes 4 for 0 and,
- * with an LDS stack, for 5 and 6, split mode applies it to the volume kernel; in
- * split mode the sampler kernel always asks for 8),
+ * wpe (waves per SIMD requested: 0, 4, 5 or 6, for the volume kernel of split mode;
+ * the fused kernel always asks for 4, the sampler kernel of split mode for 8),
  * blocks_per_cu (persistent workgroups per compute unit, 1..16). */
 int   gxy_batch_set_config(void *batch, int chunk, int stack, int wpe, int blocks_per_cu);
 int   gxy_batch_get_config(void *batch, int *chunk, int *stack, int *wpe, int *blocks_per_cu);
