@@ -90,21 +90,75 @@ __device__ __forceinline__ void block_partials(unsigned long long *v, int k0, in
 // large linear (0)
 __device__ __forceinline__ int chunk_layout(const TraceParams &P) { return sm_of(P.vv[0].vol); }
 
-// Lanes per ray of the batched marches (march_dev.h).  The lists hold random
-// rays, so with one lane per ray a wave's loads touch 64 places of the volume,
-// lines are fetched again and again (75 B per sample), and the wave marches on
-// until its longest ray ends.  Lanes of one ray share its lines.  One lane per
-// ray -> these counts: 64 mixed lists of 16K rays 15.9 -> 13.5 ms per flush,
-// 12 served requests 13.2 -> 10.4 ms (the whole batch, geometry lists included).
+// Lanes per ray of the batched marches (march_dev.h): sampler lists hold random
+// rays, and so may render lists.
 #define BG_RENDER 4
 #define BG_SAMPLE 8
 
-// The render rays of one volume chunk by the chunk's layout (MI = 1: the volume
-// has at most one isovalue).
+// Whether a render chunk is marched with one lane per ray rather than BG_RENDER.
+// Four lanes cost about 1.3 times the VALU work and pay by fetching fewer lines:
+// the lanes of a ray share them, while 64 random rays touch 64 places per load.
+// Rays that lie close together, as a camera's do, share lines without that, and
+// so does everything in a volume that the L2 holds.  So the chunk's first rays are
+// looked at: the mean distance, in voxels, of a ray to the next one in the list,
+// halfway along primary rays and at the origins of shadow and AO rays (a parent's
+// follow each other).  P.near (batch_near, runtime.cpp) has the distances, of
+// primary and other rays, at which both forms take the same time.  A chunk of up
+// to 64 / BG_RENDER rays is one round either way.
+__device__ __forceinline__ bool one_lane_chunk(const TraceParams &P, const RayList_ispc &R, const BatchChunk &ch) {
+  if (!P.vv[0].tf.bounded) return true;   // tables with infinities or NaN, as in launch_march
+  if (ch.count <= 64 / BG_RENDER) return false;
+  const bool primary = first_lane_i(gptr(R.type + ch.start)[0]) == RAY_PRIMARY;
+  const float near = P.near[primary ? 0 : 1];
+  if (near > 1e30f || near <= 0.f) return near > 0.f;
+  const int lane = threadIdx.x & 63;
+  float x = 0.f, y = 0.f, z = 0.f;
+  int in = 0;
+  if (lane < ch.count) {
+    const unsigned k = (unsigned)lane;
+    const f3 org = ray_org(R, ch.start, k), dir = ray_dir(R, ch.start, k);
+    float t0, t1;
+    box_clip(org, dir, P.blo, P.bhi, t0, t1);
+    t0 = mxf(t0, gptr(R.t + ch.start)[k]);
+    t1 = mnf(t1, gptr(R.tMax + ch.start)[k]);
+    in = t0 <= t1;
+    const float t = primary ? 0.5f * (t0 + t1) : t0;
+    const VoxRay v = vox_ray(P.vv[0].vol, org, dir);
+    x = __builtin_fmaf(t, v.b0, v.a0);
+    y = __builtin_fmaf(t, v.b1, v.a1);
+    z = __builtin_fmaf(t, v.b2, v.a2);
+  }
+  const float dx = fabsf(x - __shfl_down(x, 1, 64)), dy = fabsf(y - __shfl_down(y, 1, 64)),
+              dz = fabsf(z - __shfl_down(z, 1, 64));
+  const bool pair = lane < 63 && in && __shfl_down(in, 1, 64);
+  float sum = pair ? mxf(dx, mxf(dy, dz)) : 0.f;
+  for (int o = 32; o > 0; o >>= 1) sum += __shfl_xor(sum, o, 64);
+  const int n = __popcll(__builtin_amdgcn_ballot_w64(pair));
+  return __builtin_amdgcn_ballot_w64(sum < near * (float)n) != 0;
+}
+
+// The render rays of one volume chunk (MI = 1: the volume has at most one
+// isovalue), with one lane per ray (a wave with primary and other rays runs the
+// march of each kind) ...
 template <int SM, int MI>
-__device__ __forceinline__ unsigned long long render_chunk(const TraceParams &P, const RayList_ispc &R,
-                                                           const BatchChunk &ch, const float (*col)[3 * GXY_TF_MAX],
-                                                           const float (*op)[GXY_TF_MAX]) {
+__device__ __forceinline__ unsigned long long render_chunk_one(const TraceParams &P, const RayList_ispc &R,
+                                                               const BatchChunk &ch, const float (*col)[3 * GXY_TF_MAX],
+                                                               const float (*op)[GXY_TF_MAX]) {
+  unsigned long long n = 0;
+  const int start = ch.start;
+  NoStack stack;
+  for (int k = threadIdx.x & 63; k < ch.count; k += 64) {
+    if (gptr(R.type + start)[k] == RAY_PRIMARY) n += trace_one<1, false, SM, MI, 1>(P, R, start + k, col, op, stack);
+    else n += trace_one<1, false, SM, MI, 2>(P, R, start + k, col, op, stack);
+  }
+  return n;
+}
+// ... and with BG_RENDER lanes per ray
+template <int SM, int MI>
+__device__ __forceinline__ unsigned long long render_chunk_group(const TraceParams &P, const RayList_ispc &R,
+                                                                 const BatchChunk &ch,
+                                                                 const float (*col)[3 * GXY_TF_MAX],
+                                                                 const float (*op)[GXY_TF_MAX]) {
   unsigned long long n = 0;
   const int start = ch.start;
   for (int k = (threadIdx.x & 63) / BG_RENDER; k < ch.count; k += 64 / BG_RENDER) {
@@ -114,42 +168,43 @@ __device__ __forceinline__ unsigned long long render_chunk(const TraceParams &P,
   }
   return n;
 }
-// one ray per lane: tables with infinities or NaN (launch_march)
-template <int SM>
-__device__ __forceinline__ unsigned long long render_chunk_one(const TraceParams &P, const RayList_ispc &R,
-                                                               const BatchChunk &ch, const float (*col)[3 * GXY_TF_MAX],
-                                                               const float (*op)[GXY_TF_MAX]) {
-  unsigned long long n = 0;
-  NoStack stack;
-  for (int k = threadIdx.x & 63; k < ch.count; k += 64)
-    n += trace_one<1, false, SM, GXY_MAX_ISO>(P, R, ch.start + k, col, op, stack);
-  return n;
+// by the chunk's layout (bricked volumes with more than one isovalue take the
+// 64-bit variants, which serve any bricked copy)
+#define GXY_BY_LAYOUT(F)                                                      \
+  const int lay = chunk_layout(P);                                            \
+  const bool one = P.vv[0].nIso <= 1;                                         \
+  if (one && lay == 4) return F<4, 1>(P, R, ch, col, op);                     \
+  if (one && lay == 12) return F<12, 1>(P, R, ch, col, op);                   \
+  if (one && lay == 8) return F<8, 1>(P, R, ch, col, op);                     \
+  if (one && lay == 16) return F<16, 1>(P, R, ch, col, op);                   \
+  if (lay == 8 || lay == 16) return F<16, GXY_MAX_ISO>(P, R, ch, col, op);    \
+  if (lay == 4 || lay == 12) return F<12, GXY_MAX_ISO>(P, R, ch, col, op);    \
+  if (lay == 1) return F<1, GXY_MAX_ISO>(P, R, ch, col, op);                  \
+  return F<0, GXY_MAX_ISO>(P, R, ch, col, op);
+__device__ __forceinline__ unsigned long long render_chunk_one_any(const TraceParams &P, const RayList_ispc &R,
+                                                                   const BatchChunk &ch,
+                                                                   const float (*col)[3 * GXY_TF_MAX],
+                                                                   const float (*op)[GXY_TF_MAX]) {
+  GXY_BY_LAYOUT(render_chunk_one)
 }
-// (bricked volumes with more than one isovalue take the 64-bit variants,
-// which serve any bricked copy)
-__device__ __forceinline__ unsigned long long render_chunk_any(const TraceParams &P, const RayList_ispc &R,
-                                                               const BatchChunk &ch, int lay,
-                                                               const float (*col)[3 * GXY_TF_MAX],
-                                                               const float (*op)[GXY_TF_MAX]) {
-  if (!P.vv[0].tf.bounded) return render_chunk_one<-1>(P, R, ch, col, op);
-  const bool one = P.vv[0].nIso <= 1;
-  if (one && lay == 4) return render_chunk<4, 1>(P, R, ch, col, op);
-  if (one && lay == 12) return render_chunk<12, 1>(P, R, ch, col, op);
-  if (one && lay == 8) return render_chunk<8, 1>(P, R, ch, col, op);
-  if (one && lay == 16) return render_chunk<16, 1>(P, R, ch, col, op);
-  if (lay == 8 || lay == 16) return render_chunk<16, GXY_MAX_ISO>(P, R, ch, col, op);
-  if (lay == 4 || lay == 12) return render_chunk<12, GXY_MAX_ISO>(P, R, ch, col, op);
-  if (lay == 1) return render_chunk<1, GXY_MAX_ISO>(P, R, ch, col, op);
-  return render_chunk<0, GXY_MAX_ISO>(P, R, ch, col, op);
+__device__ __forceinline__ unsigned long long render_chunk_group_any(const TraceParams &P, const RayList_ispc &R,
+                                                                     const BatchChunk &ch,
+                                                                     const float (*col)[3 * GXY_TF_MAX],
+                                                                     const float (*op)[GXY_TF_MAX]) {
+  GXY_BY_LAYOUT(render_chunk_group)
 }
+#undef GXY_BY_LAYOUT
 
-// The sampler rays of one chunk (samples and ray passes into acc).
-__device__ __forceinline__ void sample_chunk_any(const BatchArgs &A, const TraceParams &P, const RayList_ispc &R,
-                                                 const BatchChunk &ch, int lay, float *buf, float *xyz, int *pc,
-                                                 int cap, unsigned long long *acc) {
+// The sampler rays of one chunk, every crossing of each in this launch: samples
+// and segments (counted as ray passes).
+typedef unsigned long long SampleCounts __attribute__((ext_vector_type(2)));   // (returned in registers)
+__device__ __forceinline__ SampleCounts sample_chunk(const TraceParams &P, const RayList_ispc &R, const BatchList &Ls,
+                                                     int start, int count, int ms, float *buf) {
+  float *xyz = gptr(Ls.xyz);
+  int *pc = Ls.pcount;
+  const int cap = Ls.pcap, lay = chunk_layout(P);
   ParticleBuffer B = {buf, 0};
-  const int start = ch.start, count = ch.count, ms = A.max_segments;
-  unsigned long long &ns = acc[BS_SAMPLES], &np = acc[BS_RAYS];
+  unsigned long long ns = 0, np = 0;
   if (lay == 4) sample_range<BG_SAMPLE, 4>(P, R, start, count, B, xyz, pc, cap, ms, ns, np);
   else if (lay == 8) sample_range<BG_SAMPLE, 8>(P, R, start, count, B, xyz, pc, cap, ms, ns, np);
   else if (lay == 16) sample_range<BG_SAMPLE, 16>(P, R, start, count, B, xyz, pc, cap, ms, ns, np);
@@ -157,6 +212,55 @@ __device__ __forceinline__ void sample_chunk_any(const BatchArgs &A, const Trace
   else if (lay == 1) sample_range<BG_SAMPLE, 1>(P, R, start, count, B, xyz, pc, cap, ms, ns, np);
   else sample_range<BG_SAMPLE, 0>(P, R, start, count, B, xyz, pc, cap, ms, ns, np);
   B.flush(xyz, pc, cap);
+  return SampleCounts{ns, np};
+}
+
+// A wave's transfer-function tables: an LDS slice that the kernels fill and the
+// called march below reads.
+typedef float ChunkCol[3 * GXY_TF_MAX];
+typedef float ChunkOp[GXY_TF_MAX];
+__device__ __forceinline__ ChunkCol *wave_col() {
+  __shared__ ChunkCol s_col[BWAVES];
+  return s_col + (threadIdx.x >> 6);
+}
+__device__ __forceinline__ ChunkOp *wave_op() {
+  __shared__ ChunkOp s_op[BWAVES];
+  return s_op + (threadIdx.x >> 6);
+}
+
+// The kernel that takes chunks of every kind calls these three (one call a chunk)
+// and has the one-lane march inlined.  With everything inlined it had 128 VGPRs
+// and 187 spilled SGPRs (120 and 110 so), and the march of a long ray took 5 %
+// longer.  The arguments arrive in VGPRs: uniform ones are read from the first lane.
+#define GXY_CALLED __attribute__((noinline))
+__device__ GXY_CALLED SampleCounts sample_chunk_call(const TraceParams *P, const RayList_ispc *R, const BatchList *Ls,
+                                                     int start, int count, int ms) {
+  __shared__ float s_part[BWAVES][3 * 64];
+  return sample_chunk(kconst(P), rl_global(kconst(R)), kconst(Ls), first_lane_i(start), first_lane_i(count),
+                      first_lane_i(ms), s_part[threadIdx.x >> 6]);
+}
+template <int STK>
+__device__ __forceinline__ void geom_chunk(const TraceParams &P, const RayList_ispc &R, int start, int count) {
+  constexpr int NL = STK > 0 ? STK : GXY_LDS_STACK;
+  __shared__ int s_stack[NL][GXY_BLOCK];
+  HybStack<NL, GXY_BLOCK> stack;
+  stack.base = (GXY_LDS int *)&s_stack[0][threadIdx.x];
+  const bool wide = P.model.wide == 1 || (P.model.wide == 2 && STK == 0);
+  for (int k = threadIdx.x & 63; k < count; k += 64) {
+    if (wide) trace_geom_one<decltype(stack), 4>(P, R, start, k, stack);
+    else trace_geom_one<decltype(stack), 2>(P, R, start, k, stack);
+  }
+}
+template <int STK>
+__device__ GXY_CALLED void geom_chunk_call(const TraceParams *P, const RayList_ispc *R, int start, int count) {
+  geom_chunk<STK>(kconst(P), rl_global(kconst(R)), first_lane_i(start), first_lane_i(count));
+}
+__device__ GXY_CALLED unsigned long long render_chunk_group_call(const TraceParams *P, const RayList_ispc *R, int start,
+                                                                 int count) {
+  BatchChunk ch;
+  ch.start = first_lane_i(start);
+  ch.count = first_lane_i(count);
+  return render_chunk_group_any(kconst(P), rl_global(kconst(R)), ch, wave_col(), wave_op());
 }
 
 // ------------------------------------------------------------------ pass set-up
@@ -230,19 +334,12 @@ __global__ void k_bset_count(int *ntab, int v) { *ntab = v; }
 template <int STK>
 __global__ __launch_bounds__(GXY_BLOCK) __attribute__((amdgpu_waves_per_eu(4, 8)))
 void k_btrace(BatchArgs A) {
-  __shared__ float s_part[BWAVES][3 * 64];
-  __shared__ float s_col[BWAVES][1][3 * GXY_TF_MAX];
-  __shared__ float s_op[BWAVES][1][GXY_TF_MAX];
-  constexpr int NL = STK > 0 ? STK : GXY_LDS_STACK;
-  __shared__ int s_stack[NL][GXY_BLOCK];
-  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int lane = threadIdx.x & 63;
   const int nc = *A.nin;
   unsigned long long acc[BS_COUNT];
 #pragma unroll
   for (int k = 0; k < BS_COUNT; k++) acc[k] = 0;
   int cur_tf = -1;
-  HybStack<NL, GXY_BLOCK> stack;
-  stack.base = &s_stack[0][threadIdx.x];
   for (;;) {
     int c = 0;
     if (lane == 0) c = atomicAdd(A.head, 1);
@@ -252,32 +349,29 @@ void k_btrace(BatchArgs A) {
     const BatchList &Ls = kconst(A.lists + ch.list);
     const int ds = Ls.ds, mode = Ls.mode;
     const TraceParams &P = kconst(A.ds + ds);
-    const RayList_ispc R = chunk_rays(A, ch);
-    const int lay = chunk_layout(P);
     if (mode == BM_SAMPLE) {
-      // every crossing of the ray in this launch (segments counted as ray passes)
-      float *xyz = gptr(Ls.xyz);
-      int *pc = Ls.pcount;
-      const int cap = Ls.pcap;
-      sample_chunk_any(A, P, R, ch, lay, s_part[w], xyz, pc, cap, acc);
-    } else if (P.has_model) {
-      acc[BS_RAYS] += lane < ch.count ? (ch.count - 1 - lane) / 64 + 1 : 0;
-      const bool wide = P.model.wide == 1 || (P.model.wide == 2 && STK == 0);
-      for (int k = lane; k < ch.count; k += 64) {
-        if (wide) trace_geom_one<decltype(stack), 4>(P, R, ch.start, k, stack);
-        else trace_geom_one<decltype(stack), 2>(P, R, ch.start, k, stack);
-      }
-    } else {
-      acc[BS_RAYS] += lane < ch.count ? (ch.count - 1 - lane) / 64 + 1 : 0;
-      if (ds != cur_tf) {
-        const DTF &T = P.vv[0].tf;
-        for (int k = lane; k < 3 * T.nc; k += 64) s_col[w][0][k] = T.col[k];
-        for (int k = lane; k < T.no; k += 64) s_op[w][0][k] = T.op[k];
-        wave_lds_sync();
-        cur_tf = ds;
-      }
-      acc[BS_SAMPLES] += render_chunk_any(P, R, ch, lay, s_col[w], s_op[w]);
+      const SampleCounts n = sample_chunk_call(A.ds + ds, A.rls + ch.src, A.lists + ch.list, ch.start, ch.count,
+                                               A.max_segments);
+      acc[BS_SAMPLES] += n.x;
+      acc[BS_RAYS] += n.y;
+      continue;
     }
+    acc[BS_RAYS] += lane < ch.count ? (ch.count - 1 - lane) / 64 + 1 : 0;
+    if (P.has_model) {
+      geom_chunk_call<STK>(A.ds + ds, A.rls + ch.src, ch.start, ch.count);
+      continue;
+    }
+    if (ds != cur_tf) {
+      const DTF &T = P.vv[0].tf;
+      for (int k = lane; k < 3 * T.nc; k += 64) wave_col()[0][k] = T.col[k];
+      for (int k = lane; k < T.no; k += 64) wave_op()[0][k] = T.op[k];
+      wave_lds_sync();
+      cur_tf = ds;
+    }
+    const RayList_ispc R = chunk_rays(A, ch);
+    acc[BS_SAMPLES] += one_lane_chunk(P, R, ch)
+                           ? render_chunk_one_any(P, R, ch, wave_col(), wave_op())
+                           : render_chunk_group_call(A.ds + ds, A.rls + ch.src, ch.start, ch.count);
   }
   // lane sums of the sample and ray-pass counts
   acc[BS_SAMPLES] = wave_sum_u64(acc[BS_SAMPLES]);
@@ -292,12 +386,7 @@ void k_btrace(BatchArgs A) {
 template <int KIND, int STK, int WPE>
 __global__ __launch_bounds__(GXY_BLOCK) __attribute__((amdgpu_waves_per_eu(WPE > 0 ? WPE : 1, 8)))
 void k_btrace_kind(BatchArgs A) {
-  constexpr int TFW = KIND == 0 ? BWAVES : 1;
   __shared__ float s_part[BWAVES][KIND == 2 ? 3 * 64 : 1];
-  __shared__ float s_col[TFW][1][3 * GXY_TF_MAX];
-  __shared__ float s_op[TFW][1][GXY_TF_MAX];
-  constexpr int NL = KIND != 1 ? 1 : STK > 0 ? STK : GXY_LDS_STACK;
-  __shared__ int s_stack[NL][GXY_BLOCK];
   const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int nk = A.kcount[KIND];
   const int *idx = A.kidx + (size_t)KIND * A.kcap;
@@ -305,8 +394,6 @@ void k_btrace_kind(BatchArgs A) {
 #pragma unroll
   for (int k = 0; k < BS_COUNT; k++) acc[k] = 0;
   int cur_tf = -1;
-  HybStack<NL, GXY_BLOCK> stack;
-  stack.base = &s_stack[0][threadIdx.x];
   for (;;) {
     int q = 0;
     if (lane == 0) q = atomicAdd(A.khead + KIND, 1);
@@ -318,30 +405,26 @@ void k_btrace_kind(BatchArgs A) {
     const int ds = Ls.ds;
     const TraceParams &P = kconst(A.ds + ds);
     const RayList_ispc R = chunk_rays(A, ch);
-    const int lay = chunk_layout(P);
     if (KIND == 2) {
-      float *xyz = gptr(Ls.xyz);
-      int *pc = Ls.pcount;
-      const int cap = Ls.pcap;
-      sample_chunk_any(A, P, R, ch, lay, s_part[w], xyz, pc, cap, acc);
-    } else if (KIND == 1) {
-      acc[BS_RAYS] += lane < ch.count ? (ch.count - 1 - lane) / 64 + 1 : 0;
-      const bool wide = P.model.wide == 1 || (P.model.wide == 2 && STK == 0);
-      for (int k = lane; k < ch.count; k += 64) {
-        if (wide) trace_geom_one<decltype(stack), 4>(P, R, ch.start, k, stack);
-        else trace_geom_one<decltype(stack), 2>(P, R, ch.start, k, stack);
-      }
-    } else {
-      acc[BS_RAYS] += lane < ch.count ? (ch.count - 1 - lane) / 64 + 1 : 0;
-      if (ds != cur_tf) {
-        const DTF &T = P.vv[0].tf;
-        for (int k = lane; k < 3 * T.nc; k += 64) s_col[w % TFW][0][k] = T.col[k];
-        for (int k = lane; k < T.no; k += 64) s_op[w % TFW][0][k] = T.op[k];
-        wave_lds_sync();
-        cur_tf = ds;
-      }
-      acc[BS_SAMPLES] += render_chunk_any(P, R, ch, lay, s_col[w % TFW], s_op[w % TFW]);
+      const SampleCounts n = sample_chunk(P, R, Ls, ch.start, ch.count, A.max_segments, s_part[w]);
+      acc[BS_SAMPLES] += n.x;
+      acc[BS_RAYS] += n.y;
+      continue;
     }
+    acc[BS_RAYS] += lane < ch.count ? (ch.count - 1 - lane) / 64 + 1 : 0;
+    if (KIND == 1) {
+      geom_chunk<STK>(P, R, ch.start, ch.count);
+      continue;
+    }
+    if (ds != cur_tf) {
+      const DTF &T = P.vv[0].tf;
+      for (int k = lane; k < 3 * T.nc; k += 64) wave_col()[0][k] = T.col[k];
+      for (int k = lane; k < T.no; k += 64) wave_op()[0][k] = T.op[k];
+      wave_lds_sync();
+      cur_tf = ds;
+    }
+    acc[BS_SAMPLES] += one_lane_chunk(P, R, ch) ? render_chunk_one_any(P, R, ch, wave_col(), wave_op())
+                                                : render_chunk_group_any(P, R, ch, wave_col(), wave_op());
   }
   acc[BS_SAMPLES] = wave_sum_u64(acc[BS_SAMPLES]);
   acc[BS_RAYS] = wave_sum_u64(acc[BS_RAYS]);

@@ -172,6 +172,7 @@ struct TraceParams {
   // launch covers min(n, *dn * dn_mul) rays (n is then the list's capacity)
   const int *dn;
   int dn_mul;
+  float near[2];       // batched marches: one lane per ray up to these distances between rays (batch.hip)
 };
 
 // ------------------------------------------------------------------ math

@@ -3107,6 +3107,26 @@ GXY_EXPORT int gxy_batch_update_dataset(void *b, int ds, const Visualization_isp
   return 0;
 }
 
+// Mean distances in voxels between neighbouring primary (near[0]) and other rays
+// (near[1]) up to which a batched march takes one lane per ray (one_lane_chunk,
+// batch.hip).  Measured per flush, one lane / four:
+// - random rays, 16 lists of 50 K: 4^3 bricks 64^3 1.33 / 1.41 ms, 96^3 1.71 / 1.71,
+//   128^3 2.05 / 1.97, 256^3 3.24 / 2.84, 512^3 6.4 / 4.4; linear 64^3 1.55 / 1.46,
+//   128^3 2.8 / 2.1, 512^3 10.6 / 6.1;
+// - camera rays, 8 images of 256x256 or 2 of 1024x1024 with shadow and 2 AO rays per
+//   hit, primary rays with one / four (others with four): bricks 256^3 (1.3 voxels
+//   between pixels) 2.00 / 2.13, 384^3 (1.9) 2.67 / 2.70, 512^3 (2.6) 3.38 / 3.33; linear
+//   256^3 2.39 / 2.51, 384^3 3.38 / 3.30, 512^3 4.49 / 4.04, 1024x1024 (0.65) 6.57 / 6.65;
+// - their shadow and AO rays with one / four (primary rays with one), 1024x1024:
+//   bricks 256^3 3.16 / 3.32, 384^3 3.94 / 3.87, 512^3 4.94 / 4.65; linear 64^3 1.85 /
+//   2.01, 128^3 2.79 / 2.79, 256^3 4.40 / 3.98.
+// (The mean over a camera's 8x8 tiles is 1.3 times the pixels' distance.)
+static void batch_near(const DVolume &V, float near[2]) {
+  const float edge = std::cbrt((float)V.n[0] * (float)V.n[1] * (float)V.n[2]);
+  near[0] = edge <= (V.brick ? 96.f : 48.f) ? INFINITY : V.brick ? 3.4f : 2.2f;
+  near[1] = edge <= (V.brick ? 320.f : 128.f) ? near[0] : 0.f;
+}
+
 static int batch_dataset_params(BatchObj *B, const Visualization_ispc *vis, float eps, TraceParams &P, int &depth) {
   (void)B;
   if (make_trace_params(vis, eps, P) != 0) return -1;
@@ -3117,6 +3137,7 @@ static int batch_dataset_params(BatchObj *B, const Visualization_ispc *vis, floa
   if (geometry && P.model.ncurve > 0)
     return fail("a batch dataset with path lines: path lines are traced by the per-list loop only");
   P.occlusion = (G.occlusion && geometry) ? 1 : 0;
+  if (volume) batch_near(P.vv[0].vol, P.near);
   P.hit_geom = nullptr;
   P.hit_prim = nullptr;
   P.sample_count = nullptr;

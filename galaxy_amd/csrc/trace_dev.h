@@ -189,12 +189,13 @@ __device__ __forceinline__ bool better(float t, int g, int p, const GeoHit &h) {
 // of them within the first 16).
 #define GXY_LDS_STACK 16
 #define GXY_STACK_OVER 64   // (wide_walk_fits counts on the sum of the two)
+#define GXY_LDS __attribute__((address_space(3)))
 struct NoStack {};
 template <int NL, int BS>
 struct HybStack {
   static constexpr int OVER = GXY_STACK_OVER;
   static constexpr int DEPTH = NL + OVER;
-  int *base;
+  GXY_LDS int *base;
   int over[OVER];
   __device__ __forceinline__ void put(int k, int v) {
     if (k < NL) base[k * BS] = v;
@@ -206,7 +207,7 @@ struct HybStack {
   // LDS entries free, each code is written at the top and kept by moving it.
   __device__ __forceinline__ void push4(int &sp, int c0, bool k0, int c1, bool k1, int c2, bool k2, int c3, bool k3) {
     if (__builtin_amdgcn_ballot_w64(sp > NL - 4) == 0) {
-      int *p = base + sp * BS;
+      GXY_LDS int *p = base + sp * BS;
       *p = c0;
       p += k0 ? BS : 0;
       *p = c1;

@@ -29,7 +29,7 @@ void k_geom(TraceParams P, RayList_ispc R, int n) {
   const int first = blockIdx.x * BS;
   if (first >= n || (int)threadIdx.x >= n - first) return;
   HybStack<NL, BS> stack;
-  stack.base = &s_stack[0][threadIdx.x];
+  stack.base = (GXY_LDS int *)&s_stack[0][threadIdx.x];
   trace_geom_one<HybStack<NL, BS>, W>(P, R, first, threadIdx.x, stack);
 }
 

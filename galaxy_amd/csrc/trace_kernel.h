@@ -64,7 +64,7 @@ void k_trace(TraceParams P, RayList_ispc R, int n) {
   if constexpr (GEOM) {
     __shared__ int s_stack[GXY_LDS_STACK][BS];
     HybStack<GXY_LDS_STACK, BS> stack;
-    stack.base = &s_stack[0][threadIdx.x];
+    stack.base = (GXY_LDS int *)&s_stack[0][threadIdx.x];
     if (i < n) nsamp = trace_one<NV, true, SM, MI>(P, R, i, s_col, s_op, stack);
   } else if (i < n) {
     NoStack stack;

@@ -375,3 +375,95 @@ def test_stack_check_counts_the_levels_of_the_width_asked_for(hip):
         glib.check(L.gxy_set_bvh_width(2))
     for im in images[1:]:
         assert np.abs(im - images[0]).max() <= 1e-5
+
+
+def _field(edge, seed=5, colormap=None):
+    from batch_scenes import smooth_volume
+    x = np.linspace(0.0, 1.0, 8)
+    rgb, op = workloads.VOLUME_RENDER_TF
+    vv = scenes.VolumeVisDesc(smooth_volume(edge, seed), colormap=np.c_[x, rgb].astype(f32) if colormap is None else colormap,
+                              opacitymap=np.c_[x, 4 * op].astype(f32), isovalues=np.array([0.5], f32), volume_render=True)
+    return scenes.SceneDesc(volume_vis=[vv], local_box=workloads.UNIT_BOX, global_box=workloads.UNIT_BOX)
+
+
+def _camera_list(w, h, dist=1.9, aov=40.0):
+    from galaxy_amd import lib as glib
+    hip = glib.HipBackend()
+    cam = scenes.CameraDesc((0.5 + 0.6 * dist, 0.9, 0.5 + 0.7 * dist), (0.5, 0.5, 0.5), (0, 1, 0), aov, w, h)
+    return hip.camera_rays(cam, workloads.UNIT_BOX, workloads.UNIT_BOX, 1).download()
+
+
+# one lane per ray and four: by the volume (96^3 in bricks, 48^3 linear), by the
+# distance of the rays (pixels of 0.5 and of 10 voxels, random rays), by kind (up to
+# 320^3 and 128^3 children follow their own rule), and for lists of up to 16 rays
+@pytest.mark.parametrize("edge,layout", [(40, 0), (97, 4), (64, 0), (136, 8), (136, 0)])
+@pytest.mark.parametrize("split", [0, 1])
+def test_lanes_per_ray_of_a_chunk_do_not_show(hip, edge, layout, split):
+    from galaxy_amd import batch as gb
+    from galaxy_amd import lib as glib
+    L = glib.lib()
+    built = scenes.build_scene(hip, _field(edge))
+    if layout:
+        glib.check(L.gxy_volume_set_layout(built.handles[0], layout))
+    keep = []
+    lights = lights_struct(keep)
+    lists = [(_camera_list(w, h), w, h) for w, h in ((200, 150), (16, 12), (4, 4))]
+    for n in (700, 257, 16, 1):
+        r = gb.random_rays(n, 40 + n, width=n).download()
+        lists.append((r, n, 1))
+    odd = gb.random_rays(300, 9, width=300).download()          # every kind in one list, some rays odd
+    odd["type"] = np.arange(300) % 3 + 1
+    for f, k in (("tMax", 7), ("ox", 30), ("dx", 61)):
+        odd[f][k::90] = np.inf
+        odd[f][k + 1::90] = np.nan
+    lists.append((odd, 300, 1))
+    B = gb.Batch(128)
+    ds = B.add_dataset(built)
+    B.set_lighting(lights)
+    B.set_config(128, 0, 0, 4, split)
+    fbs = []
+    for hr, w, h in lists:
+        d = glib.DeviceRays.from_host(hr)
+        fbs.append(B.add_render_list(ds, d, w, h)[1])
+        keep.append(d)
+    st = B.run(0)
+    tot = dict(rays=0, samples=0, spawned=0, terminated=0, dropped=0, kept=0)
+    nb = np.full(6, -1, np.int32)
+    for (hr, w, h), fb in zip(lists, fbs):
+        ref, s = glib.DeviceArray(16 * w * h).zero(), abi.FrameStats()
+        d = glib.DeviceRays.from_host(hr)
+        glib.check(L.gxy_process_raylist(C.byref(built.vis), C.byref(lights), hr.n, C.byref(d.ispc), nb.ctypes.data, 0.001,
+                                         1 << 30, ref.ptr, w, h, C.byref(s)))
+        a, b = fb.to_host(f32), ref.to_host(f32)
+        assert np.array_equal(np.isfinite(a), np.isfinite(b))
+        ok = np.isfinite(b)
+        assert np.abs(a - b)[ok].max() <= 1e-5, (w, h)
+        for k, f in (("rays", "ray_passes"), ("samples", "samples"), ("spawned", "secondary_rays"),
+                     ("terminated", "terminated"), ("dropped", "dropped"), ("kept", "kept")):
+            tot[k] += getattr(s, f)
+    assert {k: getattr(st, k) for k in tot} == tot
+    assert st.spawned > 1000
+
+
+@pytest.mark.parametrize("edge", [40, 64])
+@pytest.mark.parametrize("bad", [np.inf, np.nan])
+def test_unbounded_tables_in_a_batch(hip, edge, bad):
+    """A transfer function with an infinity or a NaN: one lane per ray."""
+    from galaxy_amd import batch as gb
+    from galaxy_amd import lib as glib
+    cm = np.array([[0, 0.2, 0.3, 0.4], [0.8, 0.5, 0.6, 0.7], [1.0, bad, 0.1, 0.1]], f32)
+    built = scenes.build_scene(hip, _field(edge, 6, cm))
+    keep = []
+    lights = lights_struct(keep)
+    plan = plan_of([5, 900, 4000], 1, 50)
+    B, lists = make_batch([built], lights, plan, 128)
+    B.run(0)
+    seen = 0
+    for (n, ds, seed), (l, fb) in zip(plan, lists):
+        ref, _ = plain_list(glib.lib(), built, lights, n, seed, ds)
+        got = fb.to_host(f32).reshape(-1, 4)
+        assert np.array_equal(np.isfinite(got), np.isfinite(ref))
+        ok = np.isfinite(ref)
+        seen += (~ok).sum()
+        assert np.abs(got - ref)[ok].max() <= 1e-5
+    assert seen > 10
