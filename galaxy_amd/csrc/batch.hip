@@ -243,10 +243,18 @@ template <int STK>
 __device__ __forceinline__ void geom_chunk(const TraceParams &P, const RayList_ispc &R, int start, int count) {
   constexpr int NL = STK > 0 ? STK : GXY_LDS_STACK;
   __shared__ int s_stack[NL][GXY_BLOCK];
+  GXY_LDS int *base = (GXY_LDS int *)&s_stack[0][threadIdx.x];
+  const int lane = threadIdx.x & 63;
+  if (STK > 0 && P.model.wide != 1 && P.model.depth + 2 <= STK) {
+    LdsStack<NL, GXY_BLOCK> stack;
+    stack.base = base;
+    for (int k = lane; k < count; k += 64) trace_geom_one<decltype(stack), 2>(P, R, start, k, stack);
+    return;
+  }
   HybStack<NL, GXY_BLOCK> stack;
-  stack.base = (GXY_LDS int *)&s_stack[0][threadIdx.x];
+  stack.base = base;
   const bool wide = P.model.wide == 1 || (P.model.wide == 2 && STK == 0);
-  for (int k = threadIdx.x & 63; k < count; k += 64) {
+  for (int k = lane; k < count; k += 64) {
     if (wide) trace_geom_one<decltype(stack), 4>(P, R, start, k, stack);
     else trace_geom_one<decltype(stack), 2>(P, R, start, k, stack);
   }

@@ -225,6 +225,17 @@ struct HybStack {
   }
 };
 
+// All entries in LDS: binary walks with an LDS stack setting, of trees whose depth
+// + 2 fits (the launcher's check).  Without the private part a push or pop takes no
+// branch.
+template <int NL, int BS>
+struct LdsStack {
+  static constexpr int DEPTH = NL;
+  GXY_LDS int *base;
+  __device__ __forceinline__ void put(int k, int v) { base[k * BS] = v; }
+  __device__ __forceinline__ int get(int k) const { return base[k * BS]; }
+};
+
 // Slab test of one child box against [t0, tmax] with a few ulps of slack so
 // that a primitive hit at exactly the current t still reaches its leaf.
 __device__ __forceinline__ bool child_hit(const float *lo, const float *hi, f3 o, f3 inv, float t0, float tmax,
@@ -401,7 +412,8 @@ __device__ __forceinline__ void model_trace(const DModel &M, f3 org, f3 dir, flo
         }
       }
     };
-    if (TW == 4 || (TW == 0 && M.wide)) bvh4_walk(M.tnodes4, org, inv, t0, h, stack, tleaf, any);
+    if constexpr (TW == 2) bvh_walk(M.tnodes, org, inv, t0, h, stack, tleaf, any);
+    else if (TW == 4 || M.wide) bvh4_walk(M.tnodes4, org, inv, t0, h, stack, tleaf, any);
     else bvh_walk(M.tnodes, org, inv, t0, h, stack, tleaf, any);
   }
   if (any && h.geom >= 0) return;
@@ -418,7 +430,8 @@ __device__ __forceinline__ void model_trace(const DModel &M, f3 org, f3 dir, flo
         }
       }
     };
-    if (TW == 4 || (TW == 0 && M.wide)) bvh4_walk(M.snodes4, org, inv, t0, h, stack, sleaf, any);
+    if constexpr (TW == 2) bvh_walk(M.snodes, org, inv, t0, h, stack, sleaf, any);
+    else if (TW == 4 || M.wide) bvh4_walk(M.snodes4, org, inv, t0, h, stack, sleaf, any);
     else bvh_walk(M.snodes, org, inv, t0, h, stack, sleaf, any);
   }
   if (any && h.geom >= 0) return;
@@ -441,7 +454,8 @@ __device__ __forceinline__ void model_trace(const DModel &M, f3 org, f3 dir, flo
         }
       }
     };
-    if (TW == 4 || (TW == 0 && M.wide)) bvh4_walk(M.cnodes4, org, inv, t0, h, stack, cleaf, any);
+    if constexpr (TW == 2) bvh_walk(M.cnodes, org, inv, t0, h, stack, cleaf, any);
+    else if (TW == 4 || M.wide) bvh4_walk(M.cnodes4, org, inv, t0, h, stack, cleaf, any);
     else bvh_walk(M.cnodes, org, inv, t0, h, stack, cleaf, any);
   }
 }

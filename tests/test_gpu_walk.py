@@ -185,3 +185,48 @@ def test_rays_that_skip_every_axis_find_all_children(hip, spheres):
     assert (want[1] >= 0).sum() > 100
     for a, b in zip(want, got):
         assert np.array_equal(a.view(np.int32), b.view(np.int32)), np.nonzero(a != b)[0][:5]
+
+
+def _line_scene(levels, seed):
+    """Overlapping triangles that halve in size along a line: a tree of about
+    `levels` levels, most of whose boxes a ray along the line enters."""
+    rng = np.random.default_rng([levels, seed])
+    x = 0.5 ** np.arange(levels)
+    c = np.c_[x, 0 * x, 0 * x] + 0.2 * x[:, None] * rng.uniform(-1, 1, (levels, 3))
+    v = c[:, None] + 1.5 * x[:, None, None] * rng.uniform(-0.5, 0.5, (levels, 3, 3))
+    box = ((-4.0,) * 3, (4.0,) * 3)
+    return scenes.SceneDesc(local_box=box, global_box=box, meshes=[scenes.MeshDesc(
+        v.reshape(-1, 3).astype(f32), np.arange(3 * levels, dtype=np.uint32).reshape(-1, 3))])
+
+
+def test_every_stack_holds_its_trees(hip):
+    """Trees around the depths at which an LDS stack setting still holds them, and
+    up to 60 levels: private entries, the 4-wide walk at its bound of 26 levels, and
+    the binary walk beyond it."""
+    from batch_scenes import graded_scene, rays_at_triangles
+    L = hip.L
+    depths = set()
+    scs = [_line_scene(k, s) for k in range(12, 37) for s in range(3)] + [graded_scene(s) for s in range(6)]
+    for sc in scs:
+        B = scenes.build_scene(hip, sc)
+        a, b, depth, sah = C.c_int(), C.c_int(), C.c_int(), C.c_float()
+        assert L.gxy_model_bvh_stats(B.vis.model, C.byref(a), C.byref(b), C.byref(depth), C.byref(sah)) == 0
+        depths.add(depth.value)
+        hr = rays_at_triangles(sc, 3000, 2)
+        rng = np.random.default_rng(1)
+        for f in ("oy", "oz"):                           # along the line of the triangles, both ways
+            hr[f][:600] = rng.uniform(-0.02, 0.02, 600)
+        hr["ox"][:600] = np.where(np.arange(600) % 2, 2.0, -1.0)
+        hr["dx"][:600] = np.where(np.arange(600) % 2, -1.0, 1.0)
+        for f in ("dy", "dz"):
+            hr[f][:600] = rng.uniform(-0.01, 0.01, 600)
+        hr["type"][::3] = abi.RAY_SHADOW
+        want = _closest(hip, B, hr, 2, 0)
+        assert (want[1] >= 0).sum() > 1000
+        for width, stack in ((2, 16), (2, 24), (2, 32), (4, 0)):
+            got = _closest(hip, B, hr, width, stack)
+            for x, y in zip(want, got):
+                assert np.array_equal(x.view(np.int32), y.view(np.int32)), (depth.value, width, stack)
+    for stack in (16, 24, 32):
+        assert {stack - 2, stack - 1} <= depths, sorted(depths)
+    assert max(depths) >= 55
