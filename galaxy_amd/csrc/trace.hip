@@ -338,14 +338,16 @@ static hipError_t launch_trace_nv(const TraceParams &P, const RayList_ispc &R, i
   dim3 g((n + GXY_BLOCK - 1) / GXY_BLOCK), b(GXY_BLOCK);
   bool small = true;
   for (int v = 0; v < NV; v++) small = small && P.vv[v].vol.small;
-  if (NV == 0 && P.has_model) return launch_trace_geom(P, R, n, stack, gwaves, s);
-  if (P.has_model) {
+  if constexpr (NV == 0) {
+    if (P.has_model) return launch_trace_geom(P, R, n, stack, gwaves, s);
+  } else if (P.has_model) {
     // the walk as launch_trace_geom chooses it
     TraceParams Q = P;
     if (P.model.wide == 2 && (stack != 0 || gwaves != 0)) Q.model.wide = 0;
     hipLaunchKernelGGL((k_trace<NV, true, 0, -1>), g, b, 0, s, Q, R, n);
+    return hipGetLastError();
   }
-  else if (NV == 1 && P.vv[0].vol.brick) launch_trace_bricked(P, R, n, wpe, trace_block_size(P, wpe, bs), sm_of(P.vv[0].vol), g, b, s);
+  if (NV == 1 && P.vv[0].vol.brick) launch_trace_bricked(P, R, n, wpe, trace_block_size(P, wpe, bs), sm_of(P.vv[0].vol), g, b, s);
   else if (small && wpe == 5) hipLaunchKernelGGL((k_trace<NV, false, 5, 1>), g, b, 0, s, P, R, n);
   else if (small && wpe >= 6) hipLaunchKernelGGL((k_trace<NV, false, 6, 1>), g, b, 0, s, P, R, n);
   else if (small) hipLaunchKernelGGL((k_trace<NV, false, 0, 1>), g, b, 0, s, P, R, n);
