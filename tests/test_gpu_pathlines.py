@@ -33,18 +33,22 @@ def gpu_hits(hip, built, hr):
         glib.check(L_.gxy_model_set_hit_output(built.vis.model, None, None))
 
 
-@pytest.fixture(params=[(2, 0), (4, 0), (2, 8)], ids=["binary", "wide", "binary-8-waves"])
+@pytest.fixture(params=[(2, 16, 0), (2, 0, 0), (4, 0, 0), (2, 0, 8)], ids=["binary", "default", "wide", "binary-8-waves"])
 def bvh_width(request):
-    """Runs the test with path lines walked in the binary and the 4-wide trees,
-    and in the binary tree at 8 waves per SIMD."""
+    """Runs the test with path lines walked in the binary trees (which a stack or
+    waves setting asks for, with or without 8 waves per SIMD) and in the 4-wide ones
+    (by default and by width)."""
     from galaxy_amd import lib as glib
     L_ = glib.lib()
-    saved = L_.gxy_get_bvh_width()
-    glib.check(L_.gxy_set_bvh_width(request.param[0]))
-    glib.check(L_.gxy_set_geometry_waves(request.param[1]))
+    width, stack, waves = request.param
+    saved = L_.gxy_get_bvh_width(), L_.gxy_get_geometry_stack(), L_.gxy_get_geometry_waves()
+    glib.check(L_.gxy_set_bvh_width(width))
+    glib.check(L_.gxy_set_geometry_stack(stack))
+    glib.check(L_.gxy_set_geometry_waves(waves))
     yield request.param
-    L_.gxy_set_bvh_width(saved)
-    L_.gxy_set_geometry_waves(0)
+    L_.gxy_set_bvh_width(saved[0])
+    L_.gxy_set_geometry_stack(saved[1])
+    L_.gxy_set_geometry_waves(saved[2])
 
 
 def scene_with(pl, meshes=(), box=1.5):
