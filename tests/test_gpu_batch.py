@@ -437,7 +437,7 @@ def test_lanes_per_ray_of_a_chunk_do_not_show(hip, edge, layout, split):
         a, b = fb.to_host(f32), ref.to_host(f32)
         assert np.array_equal(np.isfinite(a), np.isfinite(b))
         ok = np.isfinite(b)
-        assert np.abs(a - b)[ok].max() <= 1e-5, (w, h)
+        assert np.abs(a[ok] - b[ok]).max() <= 1e-5, (w, h)
         for k, f in (("rays", "ray_passes"), ("samples", "samples"), ("spawned", "secondary_rays"),
                      ("terminated", "terminated"), ("dropped", "dropped"), ("kept", "kept")):
             tot[k] += getattr(s, f)
@@ -465,5 +465,27 @@ def test_unbounded_tables_in_a_batch(hip, edge, bad):
         assert np.array_equal(np.isfinite(got), np.isfinite(ref))
         ok = np.isfinite(ref)
         seen += (~ok).sum()
-        assert np.abs(got - ref)[ok].max() <= 1e-5
+        assert np.abs(got[ok] - ref[ok]).max() <= 1e-5
     assert seen > 10
+
+
+@pytest.mark.parametrize("cap", [1, 63, 64, 1000])
+def test_particles_past_the_array_are_counted_not_written(datasets, hip, cap):
+    from galaxy_amd import batch as gb
+    from galaxy_amd import lib as glib
+    _, built = datasets
+    keep, runs, n, guard = [], [], 5000, 256
+    for c in (400000, cap):
+        B = gb.Batch(128)
+        B.set_lighting(lights_struct(keep))
+        d = gb.random_rays(n, 900, width=n)
+        xyz, cnt = glib.DeviceArray.from_host(np.full(3 * (c + guard), -7.0, f32)), glib.DeviceArray(4).zero()
+        glib.check(B.L.gxy_batch_add_list(B.h, B.add_dataset(built[0]), abi.BATCH_SAMPLE, n, C.byref(d.ispc), None, 0, 0,
+                                          xyz.ptr, c, cnt.ptr))
+        B.run(0)
+        runs.append((xyz.to_host(f32, 3 * (c + guard)).reshape(-1, 3), int(cnt.to_host(np.int32, 1)[0])))
+    (every, total), (some, counted) = runs
+    assert cap < total <= 400000 and counted == total
+    every = {p.tobytes() for p in every[:total]}
+    assert all(p.tobytes() in every for p in some[:cap])
+    assert (some[cap:] == -7.0).all()

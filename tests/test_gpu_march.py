@@ -165,3 +165,75 @@ def test_unbounded_tables_keep_the_one_lane_march(hip):
         a, b = _trace(hip, B, hr, 0), _trace(hip, B, hr, 16)
         for f in abi.FIELDS:
             assert np.array_equal(a[f], b[f], equal_nan=a[f].dtype == f32), f
+
+
+def _spoil(sc, seed):
+    """NaN and infinite voxels here and there."""
+    v = sc.volume_vis[0].volume
+    data = np.array(v.voxels, f32)
+    rng = np.random.default_rng(seed)
+    at = rng.random(data.shape)
+    data[at < 0.004], data[(at > 0.1) & (at < 0.104)], data[(at > 0.2) & (at < 0.204)] = np.nan, np.inf, -np.inf
+    v.voxels = data
+    return sc
+
+
+@pytest.mark.parametrize("n,edge", [(4000, 17), (65537, 33), (65537, 9)])
+def test_odd_voxels_take_the_one_lane_march(hip, n, edge):
+    """A sample of NaN or infinity counts for nothing with several lanes per ray
+    too, where it is a weight of 0 and not a branch."""
+    sc = _spoil(_volume(edge, 6), 3)
+    B = scenes.build_scene(hip, sc)
+    hr = _mixed_rays(n, 31)
+    a, b = _trace(hip, B, hr, 0), _trace(hip, B, hr, 16)
+    for f in abi.FIELDS:
+        assert np.array_equal(a[f], b[f], equal_nan=a[f].dtype == f32), f
+    plain = _volume(edge, 6)                # a second volume without odd voxels: nothing in it crosses 99
+    two = scenes.SceneDesc(volume_vis=[sc.volume_vis[0], scenes.VolumeVisDesc(plain.volume_vis[0].volume,
+                                                                              isovalues=np.array([99.0], f32))],
+                           local_box=workloads.UNIT_BOX, global_box=workloads.UNIT_BOX)
+    g, r = _sample(hip, sc, 0, _rays(n, 7)), _sample(hip, two, 0, _rays(n, 7))
+    for f in ("t", "term"):
+        assert np.array_equal(g[f], r[f], equal_nan=True), f
+
+
+@pytest.mark.parametrize("n", [1, 257, 65537, 90001])
+@pytest.mark.parametrize("edge,layout", [(9, 0), (33, 4)])
+def test_lanes_count_the_samples_of_the_one_lane_march(hip, n, edge, layout):
+    from galaxy_amd import lib as glib
+    L = glib.lib()
+    sc = _volume(edge, 6)
+    keep, stats = [], []
+    lights = scenes.make_lighting(workloads.batch_lighting(), keep)
+    nb = np.full(6, -1, np.int32)
+    saved = [C.c_int() for _ in range(3)]
+    L.gxy_get_trace_config(*[C.byref(x) for x in saved])
+    B = scenes.build_scene(hip, sc)
+    if layout:
+        glib.check(L.gxy_volume_set_layout(B.handles[0], layout))
+    hr = _rays(n, 3 + n)
+    try:
+        for kind in (0, 16):
+            glib.check(L.gxy_set_trace_config(kind, 256, 32))
+            d, fb, st = glib.DeviceRays.from_host(hr), glib.DeviceArray(16 * n).zero(), abi.FrameStats()
+            glib.check(L.gxy_process_raylist(C.byref(B.vis), C.byref(lights), n, C.byref(d.ispc), nb.ctypes.data, 0.001,
+                                             1 << 30, fb.ptr, n, 1, C.byref(st)))
+            stats.append(st.as_dict())
+    finally:
+        L.gxy_set_trace_config(*[x.value for x in saved])
+    assert stats[0] == stats[1] and (n == 1 or stats[0]["samples"] > n)
+    # two volumes count two samples a step, but one at the crossings of the first
+    counts = []
+    two = scenes.SceneDesc(volume_vis=[sc.volume_vis[0], scenes.VolumeVisDesc(sc.volume_vis[0].volume,
+                                                                              isovalues=np.array([99.0], f32))],
+                           local_box=workloads.UNIT_BOX, global_box=workloads.UNIT_BOX)
+    for s in (sc, two):
+        B2 = scenes.build_scene(hip, s)
+        if layout and s is sc:
+            glib.check(L.gxy_volume_set_layout(B2.handles[0], layout))
+        d, st, c = glib.DeviceRays.from_host(hr), abi.FrameStats(), C.c_int()
+        xyz = glib.DeviceArray(12 * (40 * n + 100))
+        glib.check(L.gxy_sample_raylist(C.byref(B2.vis), n, C.byref(d.ispc), 1 << 30, xyz.ptr, 40 * n + 100, C.byref(c),
+                                        C.byref(st)))
+        counts.append((st.samples, c.value))
+    assert counts[0][1] == counts[1][1] and counts[1][0] == 2 * counts[0][0] - counts[0][1]
