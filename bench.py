@@ -433,6 +433,9 @@ def bench_served(L, hip, nreq, seed=5, layout=0, config=None, step_rays=4_000_00
     return res
 
 
+VALU_CYCLES = 2.94      # SIMD cycles of a mean VALU instruction of the march (see valu_issue below)
+
+
 def valu_from_profile(name):
     """(VALU instructions per wave, waves per launch) of the trace kernel from
     the SQ counter line of the committed profile summary."""
@@ -553,13 +556,16 @@ def main():
                     frac=round(tfl / FP32_PEAK_TFLOPS, 5),
                     note="FP32 VALU work (no MFMA on this path); MI355X FP32 peak")
     roof["traffic"] = traffic_from_profile("trace_volume_render_traffic.txt")
-    # the bound the march actually meets: VALU issue.  A wave64 VALU instruction
-    # occupies a 16-lane SIMD for 4 cycles; 1024 SIMDs at 2.4 GHz
+    # the bound the march actually meets: VALU issue, 1024 SIMDs at 2.4 GHz.  A wave64
+    # instruction takes a SIMD 2 cycles (FP32 add, multiply and FMA, moves, 32-bit adds,
+    # logic, shifts) or 4 (compares, selects, min / max / median, conversions, 24-bit
+    # products, DPP moves, three-operand integer ones); measured with six waves per SIMD:
+    # 2.4 to 2.8 and 4.2.  The march's loop has 146 of 272 of the first kind: 2.94 a mean
     vp = valu_from_profile("trace_volume_render_traffic.txt")
     if vp and tr_n:
         ms = tr_ms / tr_n
         roof["valu_issue"] = dict(instr_per_launch=int(vp[0] * vp[1]),
-                                  frac=round(vp[0] * vp[1] * 4 / (1024 * 2.4e9 * ms * 1e-3), 4),
+                                  frac=round(vp[0] * vp[1] * VALU_CYCLES / (1024 * 2.4e9 * ms * 1e-3), 4),
                                   note="SQ_INSTS_VALU/SQ_WAVES from the committed profile x this run's launch time")
     kcfg = (C.c_int(), C.c_int(), C.c_int())
     L.gxy_get_trace_config(*[C.byref(x) for x in kcfg])
