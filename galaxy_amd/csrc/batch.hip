@@ -230,7 +230,7 @@ __device__ __forceinline__ ChunkOp *wave_op() {
 
 // The kernel that takes chunks of every kind calls these three (one call a chunk)
 // and has the one-lane march inlined.  With everything inlined it had 128 VGPRs
-// and 187 spilled SGPRs (120 and 110 so), and the march of a long ray took 5 %
+// and 187 spilled SGPRs (140 so), and the march of a long ray took 5 %
 // longer.  The arguments arrive in VGPRs: uniform ones are read from the first lane.
 #define GXY_CALLED __attribute__((noinline))
 __device__ GXY_CALLED SampleCounts sample_chunk_call(const TraceParams *P, const RayList_ispc *R, const BatchList *Ls,

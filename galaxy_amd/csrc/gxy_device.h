@@ -148,7 +148,7 @@ struct DGeomShade {
 };
 
 // The sample counter is spread over this many 64-bit counters, 128 bytes apart:
-// additions to one address complete one after another (about 15 ns each), so
+// additions to one address complete one after another (12 ns each), so
 // the waves of a large launch would queue on a single counter.
 #define GXY_COUNT_SLOTS 64
 #define GXY_COUNT_STRIDE 16

@@ -191,7 +191,7 @@ size_t      gxy_device_bytes_in_use(void);
 int         gxy_set_opacity_threshold(float alpha);
 float       gxy_get_opacity_threshold(void);
 /* Launch configuration of the volume-only trace (no reference counterpart):
- * kind 0 (default) = for one volume, 2, 4 or 16 lanes per ray by the list's size
+ * kind 0 (default) = for one volume, 1, 2, 4 or 16 lanes per ray by the list's size
  * against the length of its rays, one ray per work-item elsewhere; 15 / 16 / 17 /
  * 18 = one ray per work-item compiled for at least 5 / 6 / 7 / 8 waves per SIMD
  * (17 and 18 for one bricked volume with at most one isovalue, 16 otherwise),
@@ -202,7 +202,7 @@ float       gxy_get_opacity_threshold(void);
  * identical for every setting; galaxy_amd/autotune.py picks the fastest. */
 int         gxy_set_trace_config(int kind, int chunk, int refill);
 /* Binary BVH walk of geometry-only traces (no reference counterpart) with 16 /
- * 24 / 32 traversal stack entries in LDS (deeper entries in private memory);
+ * 24 / 32 traversal stack entries in LDS (deeper trees go on in private memory);
  * 0 (default): the walk chosen by gxy_set_bvh_width.  Results are identical for
  * every setting. */
 int         gxy_set_geometry_stack(int entries);
@@ -523,7 +523,8 @@ int   gxy_batch_set_list_seed(void *batch, int list, unsigned seed, const float 
 int   gxy_batch_remove_list(void *batch, int list);
 /* Launch configuration: chunk (rays per queue entry, 64..1024), stack (BVH traversal
  * stack: 0 = the 4-wide walk, 16/24/32 = the binary walk, or the 4-wide one with
- * BVH width 4, with that many entries in LDS; must exceed the deepest tree by 2),
+ * BVH width 4, with that many entries in LDS; must exceed the deepest tree, in levels
+ * of the BVH width asked for, by 2),
  * wpe (waves per SIMD requested: 0, 4, 5 or 6, for the volume kernel of split mode;
  * the fused kernel always asks for 4, the sampler kernel of split mode for 8),
  * blocks_per_cu (persistent workgroups per compute unit, 1..16). */
